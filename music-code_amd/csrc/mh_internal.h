@@ -110,6 +110,10 @@ int map_dense(mh_ctx *ctx, mh_map *m, const float **out);
 void ctx_release(mh_ctx *ctx);
 // Scratch buffer 'name' of at least 'bytes' bytes owned by the context.
 void *ws_get(mh_ctx *ctx, const std::string &name, size_t bytes, int *rc);
+// Ewald real-space node sums of an orthorhombic cell plus the reciprocal
+// table (mh_mapewald.hip)
+int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], const double step[3],
+                const double *recip, float *full32, double *o64, bool *done);
 // once per device (mh_ctx_create): address of mh_map_build_static's scratch
 int static_scratch_init(int device);
 

@@ -1354,7 +1354,14 @@ static int run_nodes(mh_ctx *ctx, int kind, int precision, double probe_q, const
                            axyz, ctx->type.as<int>(), ctx->q.as<double>(),
                            (const double *)nullptr, full32, o64);
     } else {
-        if (fp32)
+        bool done = false;
+        if (!slanted) {
+            int rc = ewald_nodes(ctx, probe_q, fp32 ? real_space_cutoff(ctx->ew.kappa) : 0.0, np, step, recip, full32,
+                                 o64, &done);
+            if (rc) return rc;
+        }
+        if (done) {
+        } else if (fp32)
             hipLaunchKernelGGL(k_nodes32<K_EWALD>, dim3((unsigned)nblk), dim3(NT), 0, ctx->stream, g, dt,
                                axyz, ctx->type.as<int>(), ctx->q.as<double>(),
                                recip, full32, o64);
