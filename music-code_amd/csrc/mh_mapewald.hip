@@ -7,13 +7,15 @@
 //     edge), and those whose minimum image changes inside the box, are summed
 //     node by node; the field of the others up to the real-space cutoff is
 //     smooth in the box, so it is summed at FP^3 Chebyshev points only and
-//     interpolated to the nodes axis by axis.  The nearest singularity of a
+//     interpolated to the nodes axis by axis.  Tiles of twice the edge do the
+//     same for the atoms that are far from them, and pass their polynomial on
+//     to the points of their eight tiles, where it is exact.  The nearest singularity of a
 //     far atom's field lies at 2.4 a from the box centre: the interpolation
 //     converges as 4.6^-FP, 1e-9 of V and 1e-7 of the derivatives for FP = 16,
 //     below the rounding of the FP32 values stored in the map.
 // The reference differentiates erfc exactly but evaluates it with the A&S
 // 7.1.26 fit (ewald.F90:874-916): the far field is therefore carried twice,
-// with the A&S erfc (for V) and with erfc to 1e-12 (whose interpolant is
+// with the A&S erfc (for V) and with erfc to 1e-8 (whose interpolant is
 // differentiated); the derivative terms differ from the reference's by the
 // fit's 1.5e-7 / r^2 alone.
 #include <cmath>
@@ -27,7 +29,7 @@ namespace mh {
 
 constexpr int FP = 16;            // Chebyshev points per axis
 constexpr int FPV = FP * FP * FP;
-constexpr int FDEG = 12;          // degree of the erfcx fit
+constexpr int FDEG = 9;           // degree of the erfcx fit
 constexpr int FCH = 32;           // far atoms staged per pass
 constexpr double kFarZ0 = 2.4;    // (a + R0) / a
 constexpr double kEwTokcal = 332.064;   // ewald.F90:60
@@ -39,7 +41,6 @@ struct EwP {
     int natoms;
     double step[3], L[3];
     double kappa, kappa2, pk, twoksp, charge1;
-    int refold;          // separations folded per node
     // tiles
     int SB, nt[3], nsplit;
     double rc2, r02;
@@ -78,20 +79,30 @@ __device__ __forceinline__ double ew_fold(double d, double L) {
 }
 
 // near (front, count[2 t]) and far (back, count[2 t + 1]) atoms of each tile,
-// in atom order from their end of list[t][natoms]; one workgroup per tile
-__global__ void __launch_bounds__(256) k_ew_lists(EwP p, const double *__restrict__ xyz, int *__restrict__ list,
-                                                  int *__restrict__ count) {
+// in atom order from their end of list[t][natoms]; one workgroup per tile.
+// With a parent level (tiles of twice the edge, pt tiles per axis) only the
+// atoms near the parent are looked at: the others are in its far field.
+__global__ void __launch_bounds__(256) k_ew_lists(EwP p, int ptx, int pty, const int *__restrict__ plist,
+                                                  const int *__restrict__ pcount, const double *__restrict__ xyz,
+                                                  int *__restrict__ list, int *__restrict__ count) {
     __shared__ int s_w[2][4];
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tix[3] = {t % p.nt[0], (t / p.nt[0]) % p.nt[1], t / (p.nt[0] * p.nt[1])};
     double cen[3];
     for (int d = 0; d < 3; d++) cen[d] = (double)(tix[d] * p.SB) * p.step[d] + p.half[d];
-    int nn = 0, nf = 0;
+    int nn = 0, nf = 0, total = p.natoms;
+    const int *src = nullptr;
+    if (plist) {
+        const long long pt = (tix[0] >> 1) + (long long)ptx * ((tix[1] >> 1) + (long long)pty * (tix[2] >> 1));
+        total = pcount[2 * pt];
+        src = plist + pt * p.natoms;
+    }
     int *l = list + (long long)t * p.natoms;
-    for (int a0 = 0; a0 < p.natoms; a0 += 256) {
-        const int a = a0 + tid;
+    for (int a0 = 0; a0 < total; a0 += 256) {
+        int a = a0 + tid;
         int cls = 0;  // 1 near, 2 far
-        if (a < p.natoms) {
+        if (a < total) {
+            if (src) a = src[a];
             double lb2 = 0.0;
             bool cross = false;
             for (int d = 0; d < 3; d++) {
@@ -129,6 +140,42 @@ __global__ void __launch_bounds__(256) k_ew_lists(EwP p, const double *__restric
     if (tid == 0) {
         count[2 * t] = nn;
         count[2 * t + 1] = nf;
+    }
+}
+
+// F of each tile += its parent's polynomial at the tile's points (C[o]: the
+// 16 x 16 interpolation matrix of the lower / upper half of an axis): three
+// in-place line transforms in LDS, one workgroup per tile.
+__global__ void __launch_bounds__(256) k_ew_shift(EwP p, int ptx, int pty, int psplit, long long ptiles,
+                                                  const double *__restrict__ PF, const double *__restrict__ C,
+                                                  double *__restrict__ F) {
+    __shared__ double s_f[FP][FP][FP + 1];
+    const int t = blockIdx.x, tid = threadIdx.x, i = tid & (FP - 1), j = tid >> 4;
+    const int tix[3] = {t % p.nt[0], (t / p.nt[0]) % p.nt[1], t / (p.nt[0] * p.nt[1])};
+    const long long pt = (tix[0] >> 1) + (long long)ptx * ((tix[1] >> 1) + (long long)pty * (tix[2] >> 1));
+    for (int f = 0; f < 2; f++) {
+        for (int k = 0; k < FP; k++) {
+            double v = 0.0;
+            for (int s = 0; s < psplit; s++) v += PF[((s * ptiles + pt) * 2 + f) * FPV + k * FP * FP + tid];
+            s_f[k][j][i] = v;
+        }
+        for (int d = 0; d < 3; d++) {
+            __syncthreads();
+            const double *c = C + (tix[d] & 1) * FP * FP;
+            double v[FP];
+#pragma unroll
+            for (int k = 0; k < FP; k++) v[k] = d == 0 ? s_f[j][i][k] : (d == 1 ? s_f[j][k][i] : s_f[k][j][i]);
+#pragma unroll 1
+            for (int r = 0; r < FP; r++) {
+                double o = 0.0;
+#pragma unroll
+                for (int k = 0; k < FP; k++) o = fma(c[r * FP + k], v[k], o);
+                if (d == 0) s_f[j][i][r] = o;
+                else if (d == 1) s_f[j][r][i] = o;
+                else F[((long long)t * 2 + f) * FPV + r * FP * FP + tid] += o;
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -201,18 +248,25 @@ __global__ void __launch_bounds__(256, 4) k_ew_far(EwP p, const double *__restri
 // is expanded along x and y into LDS (5 fields: V, dx, dy, value, dxdy), along
 // z in registers; the near atoms are the tile's list.  Otherwise the column
 // set has 4 groups of NZ nodes (one per wave) and every atom is summed.
-// Bound by the FP64 issue rate of the near pairs (about 70 instructions each).
+// The separations (folded) and the per-axis Gaussian factors of a staged atom
+// are formed once per axis position of the block, not per pair.
+// Bound by the FP64 issue rate of the near pairs (about 50 instructions each).
 template <int NZ, bool FAR>
-__global__ void __launch_bounds__(256, NZ == 4 ? 3 : 4) k_ew_nodes(EwP p, const double *__restrict__ xyz,
+__global__ void __launch_bounds__(256, 3) k_ew_nodes(EwP p, const double *__restrict__ xyz,
                                                      const double *__restrict__ q, const int *__restrict__ list,
                                                      const int *__restrict__ count, const double *__restrict__ F,
                                                      const double *__restrict__ M /* [2][SB][FP] */,
                                                      const double *__restrict__ recip, float *__restrict__ out32,
                                                      double *__restrict__ out64) {
+    // atoms staged per pass: per atom 8 x, 8 y and 4 NZ z entries
+    // (separation, Gaussian factor; along z with the charge)
+    constexpr int NZB = 4 * NZ, NE = 16 + NZB, NCH = 768 / NE;
     __shared__ double s_y[FAR ? 5 * FP * 64 : 1];
-    __shared__ double s_x[FAR ? 3 * 4 * FP * 8 : 1];
-    constexpr int NCH = FAR ? 32 : 128;  // atoms staged per pass (FAR: three workgroups' LDS on a CU)
-    __shared__ double4 s_at[NCH];
+    union Scratch {
+        double x[FAR ? 3 * 4 * FP * 8 : 1];
+        double2 at[NCH][NE];
+    };
+    __shared__ Scratch s_u;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int x0, y0, z0, zn, na, t = 0;
@@ -236,13 +290,7 @@ __global__ void __launch_bounds__(256, NZ == 4 ? 3 : 4) k_ew_nodes(EwP p, const 
     }
     const int x = x0 + (lane & 7), y = y0 + (lane >> 3);
     const bool valid = x < p.n[0] && y < p.n[1];
-    const double px = (double)x * p.step[0], py = (double)y * p.step[1];
-    double cen[3];  // near separations as (node - c) + fold(c - atom) when no fold can change in the box
     if (FAR) {
-        const int tx = t % p.nt[0], ty = (t / p.nt[0]) % p.nt[1], tz = t / (p.nt[0] * p.nt[1]);
-        cen[0] = (double)(tx * p.SB) * p.step[0] + p.half[0];
-        cen[1] = (double)(ty * p.SB) * p.step[1] + p.half[1];
-        cen[2] = (double)(tz * p.SB) * p.step[2] + p.half[2];
         // x and y stages, four z points at a time
         const long long tiles = (long long)p.nt[0] * p.nt[1] * p.nt[2];
         const int xo = x0 % p.SB, yo = y0 % p.SB;
@@ -276,8 +324,8 @@ __global__ void __launch_bounds__(256, NZ == 4 ? 3 : 4) k_ew_nodes(EwP p, const 
                         b = fma(m1[k], v[k], b);
                     }
                     const int o = (zc * FP + yc) * 8 + hx + i;
-                    s_x[(f == 0 ? 0 : 4 * FP * 8) + o] = a;
-                    if (f == 1) s_x[2 * 4 * FP * 8 + o] = b;
+                    s_u.x[(f == 0 ? 0 : 4 * FP * 8) + o] = a;
+                    if (f == 1) s_u.x[2 * 4 * FP * 8 + o] = b;
                 }
             }
             __syncthreads();
@@ -288,7 +336,7 @@ __global__ void __launch_bounds__(256, NZ == 4 ? 3 : 4) k_ew_nodes(EwP p, const 
 #pragma unroll 2
                 for (int k = 0; k < FP; k++) {
                     const int c = (zc * FP + k) * 8 + (lane & 7);
-                    const double a0 = s_x[c], t0 = s_x[4 * FP * 8 + c], t1 = s_x[2 * 4 * FP * 8 + c];
+                    const double a0 = s_u.x[c], t0 = s_u.x[4 * FP * 8 + c], t1 = s_u.x[2 * 4 * FP * 8 + c];
                     const double u0 = m0[k], u1 = m1[k];
                     o[0] = fma(a0, u0, o[0]);
                     o[1] = fma(t1, u0, o[1]);
@@ -337,61 +385,54 @@ __global__ void __launch_bounds__(256, NZ == 4 ? 3 : 4) k_ew_nodes(EwP p, const 
 #pragma unroll
                 for (int k = 1; k < 8; k++) S[i][k] *= sc[k];
         }
-        unsigned failed = 0;
-        double pz[NZ];
+        double rmin[NZ];
 #pragma unroll
-        for (int i = 0; i < NZ; i++) pz[i] = (double)(z0 + zl + i) * p.step[2];
+        for (int i = 0; i < NZ; i++) rmin[i] = 1.0;
 #pragma unroll 1
         for (int c0 = 0; c0 < na; c0 += NCH) {
             const int m = min(NCH, na - c0);
             __syncthreads();
-            if (tid < m) {
-                const int a = FAR ? list[(long long)t * p.natoms + c0 + tid] : c0 + tid;
-                double r[3] = {xyz[3 * a], xyz[3 * a + 1], xyz[3 * a + 2]};
-                if (FAR)
-                    for (int d = 0; d < 3; d++) r[d] = cen[d] - ew_fold(cen[d] - r[d], p.L[d]);
-                s_at[tid] = make_double4(r[0], r[1], r[2], p.charge1 * q[a]);
+            for (int w = tid; w < m * NE; w += 256) {
+                const int j = w / NE, e = w - j * NE;
+                const int a = FAR ? list[(long long)t * p.natoms + c0 + j] : c0 + j;
+                const int d = e < 8 ? 0 : (e < 16 ? 1 : 2);
+                const int node = d == 0 ? x0 + e : (d == 1 ? y0 + e - 8 : z0 + g0 * NZ + e - 16);
+                const double s = ew_fold((double)node * p.step[d] - xyz[3 * a + d], p.L[d]);
+                double g = exp(-p.kappa2 * (s * s));
+                if (d == 2) g *= p.charge1 * q[a];
+                s_u.at[j][e] = make_double2(s, g);
             }
             __syncthreads();
             if (!act) continue;
 #pragma unroll 1
             for (int j = 0; j < m; j++) {
-                const double4 at = s_at[j];
-                double sx = px - at.x, sy = py - at.y;
-                if (!FAR || p.refold) {
-                    sx = ew_fold(sx, p.L[0]);
-                    sy = ew_fold(sy, p.L[1]);
-                }
-                const double rxy = fma(sx, sx, sy * sy), sxy = sx * sy;
+                const double2 ax = s_u.at[j][lane & 7], ay = s_u.at[j][8 + (lane >> 3)];
+                const double rxy = fma(ax.x, ax.x, ay.x * ay.x), sxy = ax.x * ay.x, gxy = ax.y * ay.y;
 #pragma unroll
                 for (int i = 0; i < NZ; i++) {
-                    double sz = pz[i] - at.z;
-                    if (!FAR || p.refold) sz = ew_fold(sz, p.L[2]);
-                    double r2 = fma(sz, sz, rxy);
-                    if (r2 < kEwLowCut2) {  // the node fails; keep the arithmetic finite
-                        failed |= 1u << i;
-                        r2 = 1.0;
-                    }
+                    const double2 az = s_u.at[j][16 + wave * NZ + i];
+                    const double sz = az.x, r2 = fma(sz, sz, rxy);
+                    rmin[i] = fmin(rmin[i], r2);
                     // with u = q erfc / r, g = (2 kappa / sqrt pi) q e^{-k^2 r^2}, w = 1 / r^2:
                     // V = u; -(u + g) w s; (3 (u + g) + 2 k^2 r^2 g) w^2;
                     // -(15 (u + g) + (10 + 4 k^2 r^2) k^2 r^2 g) w^3
                     const double ri = rsq_nr(r2);
                     const double tt = rcp_nr(fma(p.pk, r2 * ri, 1.0));
                     const double k2 = p.kappa2 * r2;
-                    const double qe = at.w * exp(-k2);
+                    const double qe = gxy * az.y;
                     const double u = as_poly(tt) * (qe * ri);
                     const double gg = p.twoksp * qe;
                     const double s1 = u + gg, w = ri * ri, gk = gg * k2;
                     S[i][0] += u;
                     const double t1 = s1 * w;
-                    S[i][1] = fma(-t1, sx, S[i][1]);
-                    S[i][2] = fma(-t1, sy, S[i][2]);
+                    S[i][1] = fma(-t1, ax.x, S[i][1]);
+                    S[i][2] = fma(-t1, ay.x, S[i][2]);
                     S[i][3] = fma(-t1, sz, S[i][3]);
                     const double w2 = w * w, t2 = fma(2.0, gk, 3.0 * s1) * w2;
                     const double tz = t2 * sz;
                     S[i][4] = fma(t2, sxy, S[i][4]);
-                    S[i][5] = fma(tz, sx, S[i][5]);
-                    S[i][6] = fma(tz, sy, S[i][6]);
+                    S[i][5] = fma(tz, ax.x, S[i][5]);
+                    S[i][6] = fma(tz, ay.x, S[i][6]);
                     const double t3 = fma(fma(4.0, k2, 10.0), gk, 15.0 * s1) * (w2 * w);
                     S[i][7] = fma(-t3 * sz, sxy, S[i][7]);
                 }
@@ -405,7 +446,7 @@ __global__ void __launch_bounds__(256, NZ == 4 ? 3 : 4) k_ew_nodes(EwP p, const 
             const long long m = (long long)x + (long long)p.n[0] * ((long long)y + (long long)p.n[1] * z);
             const long long s = ((long long)x * p.n[1] + y) * p.n[2] + z;
             double o[8];
-            if ((failed >> i) & 1u) {
+            if (rmin[i] < kEwLowCut2) {
                 o[0] = kEwVeryLrg;
                 for (int k = 1; k < 8; k++) o[k] = 0.0;
             } else {
@@ -448,7 +489,7 @@ static double erfcx_host(double x) {
 }
 
 // fit of erfcx over [x0, x1] in the variable of the A&S t; false where it
-// misses 1e-11 (a range too wide for the degree)
+// misses 1e-8 (a range too wide for the degree)
 static bool fit_erfcx(double x0, double x1, EwP &p) {
     const double pp = (double)0.3275911f;
     const double ta = 1.0 / (1.0 + pp * x1), tb = 1.0 / (1.0 + pp * x0);
@@ -476,61 +517,87 @@ static bool fit_erfcx(double x0, double x1, EwP &p) {
         const double u = -1.0 + k / 32.0, ex = erfcx_host(at(u));
         double h = p.fit[FDEG];
         for (int i = FDEG - 1; i >= 0; i--) h = h * u + p.fit[i];
-        if (!(std::fabs(h - ex) <= 1e-11 * ex)) return false;
+        if (!(std::fabs(h - ex) <= 1e-8 * ex)) return false;
     }
     return true;
 }
 
-// interpolation from the Chebyshev points to nodes i = 0..SB-1 of a tile:
-// M[i][k] values, M[SB + i][k] derivatives on [-1, 1]
-static void cheb_matrices(int SB, double *M) {
-    for (int i = 0; i < SB; i++) {
-        const double xi = SB > 1 ? 2.0 * i / (SB - 1) - 1.0 : 0.0;
+// interpolation from the Chebyshev points to n positions xi on [-1, 1]:
+// M[i][k] values, D[i][k] derivatives (D may be NULL)
+static void cheb_matrix(int n, const double *xi, double *M, double *Dm) {
+    double W[FP][FP];  // series coefficient j of the point k's cardinal function
+    for (int j = 0; j < FP; j++)
+        for (int k = 0; k < FP; k++) W[j][k] = std::cos(M_PI * j * (k + 0.5) / FP) * (j == 0 ? 1.0 : 2.0) / FP;
+    for (int i = 0; i < n; i++) {
+        const double x = xi[i];
         double T[FP], D[FP];  // T_j and T_j' (recurrences)
-        T[0] = 1.0, T[1] = xi, D[0] = 0.0, D[1] = 1.0;
+        T[0] = 1.0, T[1] = x, D[0] = 0.0, D[1] = 1.0;
         for (int j = 2; j < FP; j++) {
-            T[j] = 2.0 * xi * T[j - 1] - T[j - 2];
-            D[j] = 2.0 * T[j - 1] + 2.0 * xi * D[j - 1] - D[j - 2];
+            T[j] = 2.0 * x * T[j - 1] - T[j - 2];
+            D[j] = 2.0 * T[j - 1] + 2.0 * x * D[j - 1] - D[j - 2];
         }
         for (int k = 0; k < FP; k++) {
             double v = 0.0, d = 0.0;
             for (int j = 0; j < FP; j++) {
-                const double w = std::cos(M_PI * j * (k + 0.5) / FP) * (j == 0 ? 1.0 : 2.0) / FP;
-                v += w * T[j];
-                d += w * D[j];
+                v += W[j][k] * T[j];
+                d += W[j][k] * D[j];
             }
             M[i * FP + k] = v;
-            M[(SB + i) * FP + k] = d;
+            if (Dm) Dm[i * FP + k] = d;
         }
     }
 }
 
 // Estimated FP64 instructions per node of the near + far route for tiles of
-// SB^3 nodes: 70 per near pair, 43 per far pair and point, 250 for the
-// expansion; the FP32 kernel's direct sum costs 60 per pair and 2500 for its
-// FP64 near pairs.
-static double far_cost(const EwP &p, const double rc, const double dens, int SB, double *direct) {
-    double hs = 0.0, vol = 1.0, nodes = 1.0, tiles = 1.0, e[3];
-    for (int d = 0; d < 3; d++) {
-        e[d] = (SB - 1) * p.step[d];
-        hs = std::max(hs, 0.5 * e[d]);
-        tiles *= (p.n[d] + SB - 1) / SB;
-        nodes *= p.n[d];
-        vol *= e[d];
-    }
-    const double area = 2.0 * (e[0] * e[1] + e[1] * e[2] + e[0] * e[2]);
-    const double edges = e[0] + e[1] + e[2];
-    auto grown = [&](double r) { return vol + area * r + M_PI * r * r * edges + 4.0 / 3.0 * M_PI * r * r * r; };
+// SB^3 nodes (and parents of (2 SB)^3 with two levels): 55 per near pair, 36
+// per far pair and point, 600 for the expansion; the FP32 kernel's direct sum
+// takes 60 per pair and 2500 for its FP64 near pairs.
+static double far_cost(const EwP &p, double rc, double dens, int SB, bool two, double *direct) {
     const double cell = p.L[0] * p.L[1] * p.L[2];
-    const double nall = std::min(dens * cell, dens * grown(rc));
-    // atoms whose image changes inside the box: slabs of the box's width
-    double keep = 1.0;
-    for (int d = 0; d < 3; d++)
-        if (rc + e[d] >= 0.5 * p.L[d]) keep *= std::max(0.0, 1.0 - e[d] / p.L[d]);
-    const double near0 = std::min(nall, dens * grown((kFarZ0 - 1.0) * hs));
-    const double near = near0 + (nall - near0) * (1.0 - keep);
+    auto level = [&](int sb, double &near, double &far, double within) {
+        double hs = 0.0, vol = 1.0, nodes = 1.0, tiles = 1.0, keep = 1.0, e[3];
+        for (int d = 0; d < 3; d++) {
+            e[d] = (sb - 1) * p.step[d];
+            hs = std::max(hs, 0.5 * e[d]);
+            tiles *= (p.n[d] + sb - 1) / sb;
+            nodes *= p.n[d];
+            vol *= e[d];
+            // atoms whose image changes inside the box: slabs of the box's width
+            if (rc + e[d] >= 0.5 * p.L[d]) keep *= std::max(0.0, 1.0 - e[d] / p.L[d]);
+        }
+        const double area = 2.0 * (e[0] * e[1] + e[1] * e[2] + e[0] * e[2]), edges = e[0] + e[1] + e[2];
+        auto grown = [&](double r) {
+            return std::min(dens * cell,
+                            dens * (vol + area * r + M_PI * r * r * edges + 4.0 / 3.0 * M_PI * r * r * r));
+        };
+        const double all = grown(rc);
+        near = grown((kFarZ0 - 1.0) * hs);
+        near += (all - near) * (1.0 - keep);
+        far = std::max(0.0, std::min(all, within) - near) * tiles * FPV / nodes;
+        return near;
+    };
+    double near, far, pnear = 1e300, pfar = 0.0;
+    if (two) level(2 * SB, pnear, pfar, 1e300);
+    level(SB, near, far, pnear);
     *direct = 2500.0 + 60.0 * std::min(dens * cell, dens * 4.0 / 3.0 * M_PI * rc * rc * rc * 1.25);
-    return 250.0 + 70.0 * near + 43.0 * (nall - near) * tiles * FPV / nodes;
+    return 600.0 + 55.0 * near + 36.0 * (far + pfar);
+}
+
+// tiles of SB^3 nodes of the grid in p
+static void set_tiles(EwP &p, int SB) {
+    double hmax = 0.0;
+    p.SB = SB;
+    long long tiles = 1;
+    for (int d = 0; d < 3; d++) {
+        p.nt[d] = (p.n[d] + SB - 1) / SB;
+        tiles *= p.nt[d];
+        p.half[d] = 0.5 * (SB - 1) * p.step[d];
+        p.ihalf[d] = 1.0 / p.half[d];
+        hmax = std::max(hmax, p.half[d]);
+    }
+    p.r02 = (kFarZ0 - 1.0) * hmax * (kFarZ0 - 1.0) * hmax;
+    // at least 2048 workgroups: eight waves of four on each CU
+    p.nsplit = (int)std::max<long long>(1, std::min<long long>(16, (2047 + tiles) / tiles));
 }
 
 // Real-space sums of every node of an orthorhombic cell plus the reciprocal
@@ -559,7 +626,7 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
     if (rc_real <= 0.0) {
         // four nodes per lane share the x, y parts of a pair; small grids
         // take one, for four times the waves
-        const bool four = nodes >= 64LL * 4 * 4096;
+        const bool four = nodes >= 64LL * 4 * 2048;
         const int nz = four ? 16 : 4;
         const long long nblk = (long long)((np[0] + 7) / 8) * ((np[1] + 7) / 8) * ((np[2] + nz - 1) / nz);
         if (four)
@@ -574,56 +641,81 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
         *done = true;
         return MH_OK;
     }
-    // tile size: the cheapest estimate
+    // tile size and levels: the cheapest estimate
     const double dens = p.natoms / (p.L[0] * p.L[1] * p.L[2]);
     double best = 0.0, direct = 0.0;
-    for (int SB : {16, 24, 32, 40}) {
-        bool fits = true;  // a box stays well under the single fold of the reference
-        for (int d = 0; d < 3; d++) fits = fits && (SB - 1) * step[d] < 0.45 * p.L[d];
-        if (!fits) continue;
-        const double c = far_cost(p, rc_real, dens, SB, &direct);
-        if (p.SB == 0 || c < best) best = c, p.SB = SB;
-    }
-    if (p.SB == 0 || best > 0.9 * direct) return MH_OK;
-    long long tiles = 1;
-    double hmax = 0.0, diag2 = 0.0, reach = rc_real;
-    for (int d = 0; d < 3; d++) {
-        p.nt[d] = (np[d] + p.SB - 1) / p.SB;
-        tiles *= p.nt[d];
-        p.half[d] = 0.5 * (p.SB - 1) * step[d];
-        hmax = std::max(hmax, p.half[d]);
-        diag2 += 4.0 * p.half[d] * p.half[d];
-        p.ihalf[d] = 1.0 / p.half[d];
-    }
-    const long long maxlist = 1LL << 27;  // 512 MB of list entries
-    if (tiles * p.natoms > maxlist || tiles > (1LL << 22)) return MH_OK;
-    const double R0 = (kFarZ0 - 1.0) * hmax;
+    int SB = 0;
+    bool two = false;
+    auto fits = [&](int sb) {  // a box stays well under the single fold of the reference
+        bool ok = true;
+        for (int d = 0; d < 3; d++) ok = ok && (sb - 1) * step[d] < 0.45 * p.L[d];
+        return ok;
+    };
+    for (int sb : {16, 24, 32, 40})
+        for (int lv = 0; lv < 2; lv++) {
+            if (!fits(sb << lv)) continue;
+            const double c = far_cost(p, rc_real, dens, sb, lv != 0, &direct);
+            if (SB == 0 || c < best) best = c, SB = sb, two = lv != 0;
+        }
+    if (SB == 0 || best > 0.9 * direct) return MH_OK;
     p.rc2 = rc_real * rc_real;
-    p.r02 = R0 * R0;
-    reach += std::sqrt(diag2);
-    p.refold = reach >= 0.5 * std::min(p.L[0], std::min(p.L[1], p.L[2])) ? 1 : 0;
-    if (!fit_erfcx(p.kappa * R0, p.kappa * (rc_real + std::sqrt(diag2)), p)) return MH_OK;
+    set_tiles(p, SB);
+    EwP pp = p;
+    set_tiles(pp, 2 * SB);
+    double diag2 = 0.0;
+    for (int d = 0; d < 3; d++) diag2 += 4.0 * (two ? pp : p).half[d] * (two ? pp : p).half[d];
+    const long long tiles = (long long)p.nt[0] * p.nt[1] * p.nt[2];
+    const long long ptiles = two ? (long long)pp.nt[0] * pp.nt[1] * pp.nt[2] : 0;
+    const long long maxlist = 1LL << 27;  // 512 MB of list entries
+    if ((tiles + ptiles) * p.natoms > maxlist || tiles > (1LL << 20)) return MH_OK;
+    // beyond kappa r = 5.5 the fit runs on under a Gaussian below 1e-13
+    if (!fit_erfcx(p.kappa * std::sqrt(p.r02), std::min(5.5, p.kappa * (rc_real + std::sqrt(diag2))), p)) return MH_OK;
     for (int k = 0; k < FP; k++) p.xk[k] = std::cos(M_PI * (k + 0.5) / FP);
-    // at least 2048 workgroups: eight waves of four on each CU
-    p.nsplit = (int)std::max<long long>(1, std::min<long long>(16, (2047 + tiles) / tiles));
-    std::vector<double> M(2 * (size_t)p.SB * FP);
-    cheb_matrices(p.SB, M.data());
+    std::memcpy(pp.xk, p.xk, sizeof p.xk);
+    std::memcpy(pp.fit, p.fit, sizeof p.fit);
+    pp.tc = p.tc;
+    pp.ith = p.ith;
+    // matrices: tile nodes (values, derivatives), then the two halves of a
+    // parent axis
+    std::vector<double> xi(SB), M((size_t)2 * SB * FP + 2 * FP * FP);
+    for (int i = 0; i < SB; i++) xi[i] = 2.0 * i / (SB - 1) - 1.0;
+    cheb_matrix(SB, xi.data(), M.data(), M.data() + (size_t)SB * FP);
+    double *C = M.data() + (size_t)2 * SB * FP;
+    for (int o = 0; o < 2; o++) {
+        double xs[FP];
+        // the tile's points on the parent's [-1, 1], in units of the grid step
+        const double h0 = 0.5 * (SB - 1), h1 = 0.5 * (2 * SB - 1);
+        for (int k = 0; k < FP; k++) xs[k] = (o * SB + h0 * (1.0 + p.xk[k]) - h1) / h1;
+        cheb_matrix(FP, xs, C + o * FP * FP, nullptr);
+    }
     int rc;
-    int *list = (int *)ws_get(ctx, "ewlist", sizeof(int) * tiles * p.natoms, &rc);
+    int *list = (int *)ws_get(ctx, "ewlist", sizeof(int) * (tiles + ptiles) * p.natoms, &rc);
     if (rc) return rc;
-    int *count = (int *)ws_get(ctx, "ewcount", sizeof(int) * 2 * tiles, &rc);
+    int *count = (int *)ws_get(ctx, "ewcount", sizeof(int) * 2 * (tiles + ptiles), &rc);
     if (rc) return rc;
-    double *F = (double *)ws_get(ctx, "ewfar", sizeof(double) * 2 * FPV * tiles * p.nsplit, &rc);
+    double *F = (double *)ws_get(ctx, "ewfar", sizeof(double) * 2 * FPV * (tiles * p.nsplit + ptiles * pp.nsplit), &rc);
     if (rc) return rc;
     double *dM = (double *)ws_get(ctx, "ewcheb", sizeof(double) * M.size(), &rc);
     if (rc) return rc;
     MH_HIP(hipMemcpyAsync(dM, M.data(), sizeof(double) * M.size(), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_ew_lists, dim3((unsigned)tiles), dim3(256), 0, st, p, xyz, list, count);
-    MH_HIP(hipGetLastError());
+    int *plist = two ? list + tiles * p.natoms : nullptr, *pcount = two ? count + 2 * tiles : nullptr;
+    double *PF = F + (size_t)2 * FPV * tiles * p.nsplit;
+    if (two) {
+        hipLaunchKernelGGL(k_ew_lists, dim3((unsigned)ptiles), dim3(256), 0, st, pp, 0, 0, (const int *)nullptr,
+                           (const int *)nullptr, xyz, plist, pcount);
+        hipLaunchKernelGGL(k_ew_far, dim3((unsigned)ptiles, (unsigned)pp.nsplit), dim3(256), 0, st, pp, xyz, q, plist,
+                           pcount, PF);
+        MH_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_ew_lists, dim3((unsigned)tiles), dim3(256), 0, st, p, pp.nt[0], pp.nt[1],
+                       (const int *)plist, (const int *)pcount, xyz, list, count);
     hipLaunchKernelGGL(k_ew_far, dim3((unsigned)tiles, (unsigned)p.nsplit), dim3(256), 0, st, p, xyz, q, list, count,
                        F);
+    if (two)
+        hipLaunchKernelGGL(k_ew_shift, dim3((unsigned)tiles), dim3(256), 0, st, p, pp.nt[0], pp.nt[1], pp.nsplit,
+                           ptiles, PF, dM + (size_t)2 * SB * FP, F);
     MH_HIP(hipGetLastError());
-    const int nb = p.SB / 8;
+    const int nb = SB / 8;
     hipLaunchKernelGGL((k_ew_nodes<4, true>), dim3((unsigned)(tiles * nb * nb)), dim3(256), 0, st, p, xyz, q, list,
                        count, F, dM, recip, full32, o64);
     MH_HIP(hipGetLastError());
