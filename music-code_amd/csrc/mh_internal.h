@@ -110,10 +110,19 @@ int map_dense(mh_ctx *ctx, mh_map *m, const float **out);
 void ctx_release(mh_ctx *ctx);
 // Scratch buffer 'name' of at least 'bytes' bytes owned by the context.
 void *ws_get(mh_ctx *ctx, const std::string &name, size_t bytes, int *rc);
+// Bricks of the FP32 pair kernel with a node within win of the compaction's
+// cutoff: list[0] = their number, list[1...] their indices (device memory;
+// NULL where every node came from the same route)
+struct CutBricks {
+    int b[3];
+    float cut, win;
+    int nbricks;
+    int *list;
+};
 // Ewald real-space node sums of an orthorhombic cell plus the reciprocal
 // table (mh_mapewald.hip)
 int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], const double step[3],
-                const double *recip, float *full32, double *o64, bool *done);
+                const double *recip, float *full32, double *o64, CutBricks &cb, bool *done);
 // once per device (mh_ctx_create): address of mh_map_build_static's scratch
 int static_scratch_init(int device);
 

@@ -502,15 +502,11 @@ struct LJRec {
     float4 e;       // hicut^2 (1 + 1e-6), unused
 };
 
-// at most 128 VGPRs: four waves per SIMD hide the transcendental and LDS latency
 template <int KIND>
-__global__ void __launch_bounds__(NT, 4) k_nodes32(GridP g, const PairTab *__restrict__ tab_g,
-                                                 const double *__restrict__ xyz,
-                                                 const int *__restrict__ typ,
-                                                 const double *__restrict__ qv,
-                                                 const double *__restrict__ recip,
-                                                 float *__restrict__ out32,
-                                                 double *__restrict__ out64) {
+__device__ __forceinline__ void nodes32_brick(const GridP &g, const int b, const PairTab *__restrict__ tab_g,
+                                              const double *__restrict__ xyz, const int *__restrict__ typ,
+                                              const double *__restrict__ qv, const double *__restrict__ recip,
+                                              float *__restrict__ out32, double *__restrict__ out64) {
     // culled atoms, one LDS record per atom: (x, y, z relative to the brick
     // centre, p0) with p0 = hicut^2 (1 - 1e-6) for LJ and the charge product
     // for Ewald; LJ adds its pair coefficients and hicut^2 (1 + 1e-6) with the
@@ -530,7 +526,6 @@ __global__ void __launch_bounds__(NT, 4) k_nodes32(GridP g, const PairTab *__res
         __syncthreads();
     }
     const int nbx = (g.nx + BX - 1) / BX, nby = (g.ny + BY - 1) / BY;
-    const int b = blockIdx.x;
     const int bx = b % nbx, by = (b / nbx) % nby, bz = b / (nbx * nby);
     // lanes run along z first: the node values are stored in the map's scan
     // order (z fastest), four consecutive z of a column per 128-byte line
@@ -757,6 +752,33 @@ __global__ void __launch_bounds__(NT, 4) k_nodes32(GridP g, const PairTab *__res
     }
 }
 
+// at most 128 VGPRs: four waves per SIMD hide the transcendental and LDS latency
+template <int KIND>
+__global__ void __launch_bounds__(NT, 4) k_nodes32(GridP g, const PairTab *__restrict__ tab_g,
+                                                 const double *__restrict__ xyz,
+                                                 const int *__restrict__ typ,
+                                                 const double *__restrict__ qv,
+                                                 const double *__restrict__ recip,
+                                                 float *__restrict__ out32,
+                                                 double *__restrict__ out64) {
+    nodes32_brick<KIND>(g, blockIdx.x, tab_g, xyz, typ, qv, recip, out32, out64);
+}
+
+// The listed bricks only: those with a node so close to the compaction's
+// cutoff that the far-field route could put it on the other side
+__global__ void __launch_bounds__(NT, 4) k_nodes32_list(GridP g, const int *__restrict__ nlist,
+                                                      const int *__restrict__ list,
+                                                      const double *__restrict__ xyz,
+                                                      const double *__restrict__ qv,
+                                                      const double *__restrict__ recip,
+                                                      float *__restrict__ out32, double *__restrict__ out64) {
+    const int n = *nlist;
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        nodes32_brick<K_EWALD>(g, list[i], nullptr, xyz, nullptr, qv, recip, out32, out64);
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------ Ewald reciprocal part
 // Parity mode: V(r) = Re sum_k c_k e^{ik.r}, with c_k = s_k + i si_k
 // (ewald_skwaldHOT, ewald.F90:966-1005: realPart = s cos - si sin, which
@@ -868,60 +890,92 @@ __global__ void __launch_bounds__(256) k_recip_xy(int side, int nx, int ny, int 
 // each below-cutoff node takes 1 + (number of neighbours it owns) indices,
 // assigned by an exclusive prefix sum in scan order.  Scan index
 // s = (i*ny + j)*nz + k is also the ptr layout index.
+//
+// Everything but the records themselves is bit rows: word w of row (i, j)
+// holds the nodes k = 64 w .. 64 w + 63, W words a row, and the 26 neighbour
+// tests of 64 nodes are shifts of whole words.  Per word:
+//   below      nodes under the cutoff
+//   own[5]     bit planes of each node's code: the direction of its owner,
+//              (di + 1) 9 + (dj + 1) 3 + (dk + 1); 13 = none (or below)
+//   num[5]     bit planes of the number of neighbours each node owns
+//   cnt, base  indices its nodes take, their exclusive prefix sum
+// One lane per node over byte and int32 arrays (26 neighbour loads in three
+// kernels) took 2.9 ms of the 334^3 charged map.  Bound by HBM: V of every
+// node is read once, each kept record read and written once.
+typedef unsigned long long u64;
+constexpr int kSelf = 13;
+
 __device__ __forceinline__ int wrapi(int a, int n) { return a >= n ? 0 : (a < 0 ? n - 1 : a); }
 
-__global__ void k_below(long long n, int nx, int ny, int nz, const float *__restrict__ full,
-                        float cut, uint8_t *__restrict__ below) {
-    long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    below[s] = full[8 * s] < cut ? 1 : 0;
+__global__ void __launch_bounds__(256) k_below(int rows, int nz, int W, const float *__restrict__ full, float cut,
+                                               u64 *__restrict__ below) {
+    const long long word = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (word >= (long long)rows * W) return;
+    const long long row = word / W;
+    const int z = (int)(word - row * W) * 64 + lane;
+    const bool b = z < nz && full[8 * (row * nz + z)] < cut;
+    const u64 m = __ballot(b);
+    if (lane == 0) below[word] = m;
 }
 
-__global__ void k_owner(long long n, int nx, int ny, int nz, const uint8_t *__restrict__ below,
-                        int32_t *__restrict__ owner) {
-    long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    int k = (int)(s % nz), j = (int)((s / nz) % ny), i = (int)(s / ((long long)nz * ny));
-    long long best = -1;
-    if (!below[s]) {
-        for (int ii = -1; ii <= 1; ii++)
-            for (int jj = -1; jj <= 1; jj++)
-                for (int kk = -1; kk <= 1; kk++) {
-                    if (!ii && !jj && !kk) continue;
-                    long long t = ((long long)wrapi(i + ii, nx) * ny + wrapi(j + jj, ny)) * nz + wrapi(k + kk, nz);
-                    if (below[t] && (best < 0 || t < best)) best = t;
-                }
-    }
-    owner[s] = (int32_t)best;
+// neighbour offset q = 0, 1, 2 of coordinate a in the order of the wrapped index
+__device__ __forceinline__ int scan_off(int q, int a, int n) {
+    if (a == 0) return q == 2 ? -1 : q;          // 0, 1, n - 1
+    if (a == n - 1) return q == 0 ? 1 : q - 2;   // 0, n - 2, n - 1
+    return q - 1;
 }
 
-__global__ void __launch_bounds__(256) k_count(long long n, int nx, int ny, int nz,
-                                               const uint8_t *__restrict__ below,
-                                               const int32_t *__restrict__ owner,
-                                               int32_t *__restrict__ cnt,
-                                               unsigned long long *__restrict__ partial) {
-    __shared__ unsigned long long sred[3][4];
-    long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    int c = 0;
-    unsigned long long tb = 0, tn = 0, tr = 0;
-    if (s < n) {
-        int k = (int)(s % nz), j = (int)((s / nz) % ny), i = (int)(s / ((long long)nz * ny));
-        if (below[s]) {
-            c = 1;
-            tb = 1;
-            for (int ii = -1; ii <= 1; ii++)
-                for (int jj = -1; jj <= 1; jj++)
-                    for (int kk = -1; kk <= 1; kk++) {
-                        if (!ii && !jj && !kk) continue;
-                        long long t = ((long long)wrapi(i + ii, nx) * ny + wrapi(j + jj, ny)) * nz + wrapi(k + kk, nz);
-                        if (!below[t] && owner[t] == s) c++;
-                    }
-        } else {
-            long long o = owner[s];
-            if (o >= 0) tn = 1;
-            if (o < 0 || o > s) tr = 1;  // still unassigned when the scan reaches s
+// owner codes of the 64 nodes of a word, one lane per word, and the tallies
+// (below, owned, still unassigned when the scan reaches the node)
+__global__ void __launch_bounds__(256) k_owner(int nx, int ny, int nz, int W, long long words,
+                                               const u64 *__restrict__ below, u64 *__restrict__ own,
+                                               u64 *__restrict__ partial) {
+    __shared__ u64 sred[3][4];
+    const long long word = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    u64 tb = 0, tn = 0, tr = 0;
+    if (word < words) {
+        const int row = (int)(word / W), w = (int)(word - (long long)row * W);
+        const int i = row / ny, j = row - i * ny;
+        const int lb = (nz - 1) & 63;
+        const bool w0 = w == 0, wl = w == W - 1;
+        const u64 valid = wl ? (~0ull >> (63 - lb)) : ~0ull;
+        const u64 me = below[word];
+        u64 avail = ~me & valid, late = 0, p[5] = {0, 0, 0, 0, 0};
+        for (int a = 0; a < 3; a++) {
+            const int di = scan_off(a, i, nx), ii = wrapi(i + di, nx);
+            for (int b = 0; b < 3; b++) {
+                const int dj = scan_off(b, j, ny), r = ii * ny + wrapi(j + dj, ny);
+                const u64 *R = below + (long long)r * W;
+                const u64 c = R[w], pv = w0 ? 0ull : R[w - 1], nv = wl ? 0ull : R[w + 1];
+                const u64 zfirst = wl ? (R[0] & 1ull) : 0ull, zlast = w0 ? ((R[W - 1] >> lb) & 1ull) : 0ull;
+                const int base = (di + 1) * 9 + (dj + 1) * 3;
+                const u64 after = r > row ? ~0ull : 0ull, same = r == row ? ~0ull : 0ull;
+                auto take = [&](u64 m, int code, u64 is_late) {
+                    avail &= ~m;
+                    late |= m & is_late;
+#pragma unroll
+                    for (int q = 0; q < 5; q++)
+                        if ((code >> q) & 1) p[q] |= m;
+                };
+                // the row's nodes in index order: z = 0 of the last node's
+                // wrap, k - 1, k, k + 1, the wrap of the first node
+                if (wl) take(avail & (zfirst << lb), base + 2, after);
+                take(avail & ((c << 1) | (pv >> 63)), base, after);
+                take(avail & c, base + 1, after);
+                take(avail & ((c >> 1) | (nv << 63)), base + 2, after | same);
+                if (w0) take(avail & zlast, base, after | same);
+            }
         }
-        cnt[s] = c;
+        const u64 none = ~(~me & valid) | avail;
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            if ((kSelf >> q) & 1) p[q] |= none;
+            own[q * words + word] = p[q];
+        }
+        tb = __popcll(me);
+        tn = __popcll(~none);
+        tr = __popcll(avail) + __popcll(late);
     }
     // block reduction, one partial per block (no global atomics)
     for (int off = 32; off > 0; off >>= 1) {
@@ -937,14 +991,119 @@ __global__ void __launch_bounds__(256) k_count(long long n, int nx, int ny, int 
     }
     __syncthreads();
     if (threadIdx.x < 3) {
-        unsigned long long v = 0;
+        u64 v = 0;
         for (int w = 0; w < 4; w++) v += sred[threadIdx.x][w];
         partial[3 * (long long)blockIdx.x + threadIdx.x] = v;
     }
 }
 
-__global__ void __launch_bounds__(1024) k_tally(long long nblk, const unsigned long long *__restrict__ partial,
-                                                unsigned long long *__restrict__ tallies) {
+// nodes of a word whose neighbour in direction d is theirs: the neighbour's
+// code points back, 26 - d (bits past the row's end are undefined: the caller
+// keeps those of below-cutoff nodes)
+__device__ __forceinline__ u64 owned_mask(const u64 *__restrict__ own, long long words, int nx, int ny, int nz, int W,
+                                          int i, int j, int w, int d) {
+    const int di = d / 9 - 1, dj = (d / 3) % 3 - 1, dk = d % 3 - 1, code = 26 - d;
+    const long long r = (long long)(wrapi(i + di, nx) * ny + wrapi(j + dj, ny)) * W;
+    auto eq = [&](int x) {
+        u64 m = ~0ull;
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            const u64 v = own[q * words + r + x];
+            m &= ((code >> q) & 1) ? v : ~v;
+        }
+        return m;
+    };
+    const int lb = (nz - 1) & 63;
+    const u64 c = eq(w);
+    if (dk == 0) return c;
+    // the neighbouring word that the shift borrows from, or the row's other end
+    if (dk > 0) return w == W - 1 ? (c >> 1) | ((eq(0) & 1ull) << lb) : (c >> 1) | (eq(w + 1) << 63);
+    return w == 0 ? (c << 1) | ((eq(W - 1) >> lb) & 1ull) : (c << 1) | (eq(w - 1) >> 63);
+}
+
+// owned neighbours of the 64 nodes of a word (bit-sliced sums) and the
+// indices they take, one lane per word
+__global__ void __launch_bounds__(256) k_count(int nx, int ny, int nz, int W, long long words,
+                                               const u64 *__restrict__ below, const u64 *__restrict__ own,
+                                               u64 *__restrict__ num, int32_t *__restrict__ cnt) {
+    const long long word = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (word >= words) return;
+    const int row = (int)(word / W), w = (int)(word - (long long)row * W);
+    const int i = row / ny, j = row - i * ny;
+    const u64 me = below[word];
+    u64 n[5] = {0, 0, 0, 0, 0};
+    if (me) {
+        for (int d = 0; d < 27; d++) {
+            if (d == kSelf) continue;
+            u64 c = owned_mask(own, words, nx, ny, nz, W, i, j, w, d) & me;
+#pragma unroll
+            for (int q = 0; q < 5; q++) {
+                const u64 t = n[q] & c;
+                n[q] ^= c;
+                c = t;
+            }
+        }
+    }
+    int total = __popcll(me);
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        num[q * words + word] = n[q];
+        total += __popcll(n[q]) << q;
+    }
+    cnt[word] = total;
+}
+
+// numbers and records of a word's nodes and of the neighbours they own, one
+// wave per word (a lane per node; lane d < 27 forms the mask of direction d)
+__global__ void __launch_bounds__(256) k_assign(int nx, int ny, int nz, int W, long long words,
+                                                const u64 *__restrict__ below, const u64 *__restrict__ own,
+                                                const u64 *__restrict__ num, const int32_t *__restrict__ base,
+                                                const float *__restrict__ full, int32_t *__restrict__ ptr,
+                                                float *__restrict__ cvals) {
+    const long long word = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (word >= words) return;
+    const int row = (int)(word / W), w = (int)(word - (long long)row * W);
+    const int i = row / ny, j = row - i * ny;
+    const int z = w * 64 + lane;
+    const u64 me = below[word];
+    u64 mask = lane < 27 ? owned_mask(own, words, nx, ny, nz, W, i, j, w, lane) : 0ull;
+    if (lane != kSelf) mask &= me;
+    auto of = [&](int d) {
+        return (u64)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)mask, d) |
+               ((u64)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(mask >> 32), d) << 32);
+    };
+    auto lower = [&](u64 m) {  // bits of m below the lane's
+        return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    };
+    const bool mine = (me >> lane) & 1ull;
+    if (z < nz && !mine && ((of(kSelf) >> lane) & 1ull)) ptr[(long long)row * nz + z] = 0;
+    if (!me) return;
+    long long idx = (long long)base[word] + lower(me);
+#pragma unroll
+    for (int q = 0; q < 5; q++) idx += (long long)lower(num[q * words + word]) << q;
+    auto put = [&](long long t, long long k) {
+        ptr[t] = (int32_t)(k + 1);
+        const float4 *src = reinterpret_cast<const float4 *>(full + 8 * t);
+        float4 *dst = reinterpret_cast<float4 *>(cvals + 8 * k);
+        const float4 a = src[0], b = src[1];
+        dst[0] = a;
+        dst[1] = b;
+    };
+    if (mine) put((long long)row * nz + z, idx);
+    for (int d = 0; d < 27; d++) {
+        const u64 m = of(d);
+        if (d == kSelf || m == 0) continue;
+        if ((m >> lane) & 1ull) {
+            const int a = wrapi(i + d / 9 - 1, nx), b = wrapi(j + (d / 3) % 3 - 1, ny), c = wrapi(z + d % 3 - 1, nz);
+            idx++;
+            put(((long long)a * ny + b) * nz + c, idx);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(1024) k_tally(long long nblk, const u64 *__restrict__ partial,
+                                                u64 *__restrict__ tallies) {
     __shared__ unsigned long long sh[3][1024];
     unsigned long long v[3] = {0, 0, 0};
     for (long long b = threadIdx.x; b < nblk; b += 1024)
@@ -984,64 +1143,24 @@ __global__ void k_scan_add(long long n, int32_t *__restrict__ out, const int32_t
     if (i < n) out[i] += boff[blockIdx.x];
 }
 
-__global__ void k_assign(long long n, int nx, int ny, int nz, const uint8_t *__restrict__ below,
-                         const int32_t *__restrict__ owner, const int32_t *__restrict__ base,
-                         const float *__restrict__ full, int32_t *__restrict__ ptr,
-                         float *__restrict__ cvals) {
-    long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    int k = (int)(s % nz), j = (int)((s / nz) % ny), i = (int)(s / ((long long)nz * ny));
-    if (below[s]) {
-        long long idx = base[s];
-        ptr[s] = (int32_t)(idx + 1);
-        const float4 *src = reinterpret_cast<const float4 *>(full + 8 * s);
-        float4 *dst = reinterpret_cast<float4 *>(cvals + 8 * idx);
-        dst[0] = src[0];
-        dst[1] = src[1];
-        for (int ii = -1; ii <= 1; ii++)
-            for (int jj = -1; jj <= 1; jj++)
-                for (int kk = -1; kk <= 1; kk++) {
-                    if (!ii && !jj && !kk) continue;
-                    int a = wrapi(i + ii, nx), bb = wrapi(j + jj, ny), c = wrapi(k + kk, nz);
-                    long long t = ((long long)a * ny + bb) * nz + c;
-                    if (!below[t] && owner[t] == s) {
-                        idx++;
-                        ptr[t] = (int32_t)(idx + 1);
-                        const float4 *s2 = reinterpret_cast<const float4 *>(full + 8 * t);
-                        float4 *d2 = reinterpret_cast<float4 *>(cvals + 8 * idx);
-                        d2[0] = s2[0];
-                        d2[1] = s2[1];
-                    }
-                }
-    } else if (owner[s] < 0) {
-        ptr[s] = 0;
-    }
-}
-
-__global__ void k_fill_i32(long long n, int32_t v, int32_t *__restrict__ p) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-__global__ void k_fill_u64(int n, unsigned long long *__restrict__ p) {
-    if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
-}
-
 // Scratch of mh_map_build_static: a file-scope device array (one copy per
 // device, held until the process ends), carved as below; its device address
 // per device comes from hipGetSymbolAddress (the array's name is a host
 // stand-in, not a device address).
 constexpr long long kStaticMaxNodes = 1LL << 21;
 constexpr size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
-constexpr long long kStaticBlocks256 = kStaticMaxNodes / 256;
-constexpr long long kStaticScan0 = kStaticMaxNodes / 1024 + 1;
+// words of the bit rows: at most one per three nodes (a row has three at least)
+constexpr long long kStaticMaxWords = kStaticMaxNodes / 3 + 1;
+constexpr long long kStaticBlocks256 = kStaticMaxWords / 256 + 1;
+constexpr long long kStaticScan0 = kStaticMaxWords / 1024 + 2;
 constexpr size_t kOffFull32 = 0;
 constexpr size_t kOffBelow = kOffFull32 + al256(sizeof(float) * 8 * kStaticMaxNodes);
-constexpr size_t kOffOwner = kOffBelow + al256(kStaticMaxNodes);
-constexpr size_t kOffCnt = kOffOwner + al256(sizeof(int32_t) * kStaticMaxNodes);
-constexpr size_t kOffBase = kOffCnt + al256(sizeof(int32_t) * kStaticMaxNodes);
-constexpr size_t kOffPartial = kOffBase + al256(sizeof(int32_t) * kStaticMaxNodes);
-constexpr size_t kOffTallies = kOffPartial + al256(sizeof(unsigned long long) * 3 * kStaticBlocks256);
+constexpr size_t kOffOwn = kOffBelow + al256(sizeof(u64) * kStaticMaxWords);
+constexpr size_t kOffNum = kOffOwn + al256(sizeof(u64) * 5 * kStaticMaxWords);
+constexpr size_t kOffCnt = kOffNum + al256(sizeof(u64) * 5 * kStaticMaxWords);
+constexpr size_t kOffBase = kOffCnt + al256(sizeof(int32_t) * kStaticMaxWords);
+constexpr size_t kOffPartial = kOffBase + al256(sizeof(int32_t) * kStaticMaxWords);
+constexpr size_t kOffTallies = kOffPartial + al256(sizeof(u64) * 3 * kStaticBlocks256);
 constexpr size_t kOffScan = kOffTallies + 256;
 constexpr size_t kScanLevelBytes = al256(sizeof(int32_t) * kStaticScan0);
 constexpr size_t kOffPairTab = kOffScan + 8 * kScanLevelBytes;
@@ -1104,64 +1223,50 @@ static int scan_exclusive_b(mh_ctx *ctx, int level, long long n, const int32_t *
     return MH_OK;
 }
 
-static int scan_exclusive(mh_ctx *ctx, long long n, const int32_t *in, int32_t *out, int64_t *total) {
-    int32_t *bsum[4] = {nullptr, nullptr, nullptr, nullptr}, *boff[4] = {nullptr, nullptr, nullptr, nullptr};
-    long long m = n;
-    int rc = MH_OK;
-    for (int l = 0; l < 4 && m > 0; l++) {
-        long long nb = (m + SCAN_B - 1) / SCAN_B;
-        std::string lv = std::to_string(l);
-        bsum[l] = (int32_t *)ws_get(ctx, "scan_bsum" + lv, sizeof(int32_t) * (nb + 1), &rc);
-        if (rc) return rc;
-        boff[l] = (int32_t *)ws_get(ctx, "scan_boff" + lv, sizeof(int32_t) * (nb + 1), &rc);
-        if (rc) return rc;
-        if (nb == 1) break;
-        m = nb;
-    }
-    return scan_exclusive_b(ctx, 0, n, in, out, bsum, boff, total);
-}
-
 // compaction buffers (pmap_compact restated for the device)
 struct CompactBufs {
-    uint8_t *below;
-    int32_t *owner, *cnt, *base;
-    unsigned long long *tallies, *partial;
+    u64 *below, *own, *num;
+    int32_t *cnt, *base;
+    u64 *tallies, *partial;
+    int32_t *bsum[4], *boff[4];  // levels of the prefix sum
 };
 
+// words of the bit rows of a grid
+static long long compact_words(const int np[3]) { return (long long)np[0] * np[1] * ((np[2] + 63) / 64); }
+
 // below / owner / count / tallies / scan: returns the number of tabulated
-// records (host) and leaves ptr zeroed
-static int compact_count(mh_ctx *ctx, const int np[3], long long nodes, const float *full32, float cut,
-                         const CompactBufs &b, int32_t *const *bsum, int32_t *const *boff, int32_t *ptr,
+// records (host)
+static int compact_count(mh_ctx *ctx, const int np[3], const float *full32, float cut, const CompactBufs &b,
                          int64_t *total) {
     hipStream_t st = ctx->stream;
-    unsigned gb = (unsigned)((nodes + 255) / 256);
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, st, 4, b.tallies);
-    hipLaunchKernelGGL(k_fill_i32, dim3(gb), dim3(256), 0, st, nodes, 0, ptr);
-    hipLaunchKernelGGL(k_below, dim3(gb), dim3(256), 0, st, nodes, np[0], np[1], np[2], full32, cut, b.below);
-    hipLaunchKernelGGL(k_owner, dim3(gb), dim3(256), 0, st, nodes, np[0], np[1], np[2], b.below, b.owner);
-    hipLaunchKernelGGL(k_count, dim3(gb), dim3(256), 0, st, nodes, np[0], np[1], np[2], b.below, b.owner, b.cnt,
-                       b.partial);
-    hipLaunchKernelGGL(k_tally, dim3(1), dim3(1024), 0, st, (long long)gb, b.partial, b.tallies);
+    const int W = (np[2] + 63) / 64;
+    const long long words = compact_words(np);
+    const unsigned gw = (unsigned)((words + 255) / 256), gq = (unsigned)((words + 3) / 4);
+    hipLaunchKernelGGL(k_below, dim3(gq), dim3(256), 0, st, np[0] * np[1], np[2], W, full32, cut, b.below);
+    hipLaunchKernelGGL(k_owner, dim3(gw), dim3(256), 0, st, np[0], np[1], np[2], W, words, b.below, b.own, b.partial);
+    hipLaunchKernelGGL(k_count, dim3(gw), dim3(256), 0, st, np[0], np[1], np[2], W, words, b.below, b.own, b.num,
+                       b.cnt);
+    hipLaunchKernelGGL(k_tally, dim3(1), dim3(1024), 0, st, (long long)gw, b.partial, b.tallies);
     if (hipGetLastError() != hipSuccess) {
         set_error("map compaction: kernel launch failed");
         return MH_EHIP;
     }
-    if (bsum) return scan_exclusive_b(ctx, 0, nodes, b.cnt, b.base, bsum, boff, total);
-    return scan_exclusive(ctx, nodes, b.cnt, b.base, total);
+    return scan_exclusive_b(ctx, 0, words, b.cnt, b.base, b.bsum, b.boff, total);
 }
 
 // numbering and record copies; counts = acceptCut, acceptNeighbor, naccept, reject
-static int compact_assign(mh_ctx *ctx, const int np[3], long long nodes, const float *full32,
-                          const CompactBufs &b, int32_t *ptr, float *vals, int64_t total, int64_t counts[4]) {
+static int compact_assign(mh_ctx *ctx, const int np[3], const float *full32, const CompactBufs &b, int32_t *ptr,
+                          float *vals, int64_t total, int64_t counts[4]) {
     hipStream_t st = ctx->stream;
-    unsigned gb = (unsigned)((nodes + 255) / 256);
-    hipLaunchKernelGGL(k_assign, dim3(gb), dim3(256), 0, st, nodes, np[0], np[1], np[2], b.below, b.owner, b.base,
-                       full32, ptr, vals);
+    const int W = (np[2] + 63) / 64;
+    const long long words = compact_words(np);
+    hipLaunchKernelGGL(k_assign, dim3((unsigned)((words + 3) / 4)), dim3(256), 0, st, np[0], np[1], np[2], W, words,
+                       b.below, b.own, b.num, b.base, full32, ptr, vals);
     if (hipGetLastError() != hipSuccess) {
         set_error("map compaction: assign kernel launch failed");
         return MH_EHIP;
     }
-    unsigned long long t[4];
+    u64 t[3];
     if (hipMemcpyAsync(t, b.tallies, sizeof t, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess) {
         set_error("map compaction: synchronisation failed");
@@ -1246,7 +1351,7 @@ static double real_space_cutoff(double kappa) {
 // values into full32 (and FP64 into o64 when not NULL); dt is device memory
 // for the pair table
 static int run_nodes(mh_ctx *ctx, int kind, int precision, double probe_q, const int np[3], const double step[3],
-                     PairTab *dt, float *full32, double *o64, bool timed) {
+                     PairTab *dt, float *full32, double *o64, float cut, bool timed) {
     const LJTable &lj = ctx->lj;
     double *recip = nullptr;
     // pair tables
@@ -1356,9 +1461,14 @@ static int run_nodes(mh_ctx *ctx, int kind, int precision, double probe_q, const
     } else {
         bool done = false;
         if (!slanted) {
+            // the two FP32 routes agree within 1e-5 of max(|V|, 1 kcal/mol)
+            CutBricks cb{{BX, BY, BZ}, cut, 1e-5f * fmaxf(fabsf(cut), 1.0f), (int)nblk, nullptr};
             int rc = ewald_nodes(ctx, probe_q, fp32 ? real_space_cutoff(ctx->ew.kappa) : 0.0, np, step, recip, full32,
-                                 o64, &done);
+                                 o64, cb, &done);
             if (rc) return rc;
+            if (done && cb.list)
+                hipLaunchKernelGGL(k_nodes32_list, dim3(512), dim3(NT), 0, ctx->stream, g, cb.list, cb.list + 1, axyz,
+                                   ctx->q.as<double>(), recip, full32, o64);
         }
         if (done) {
         } else if (fp32)
@@ -1437,35 +1547,48 @@ extern "C" int mh_map_build(mh_ctx *ctx, int kind, int precision, double probe_q
     double *o64 = want64 ? full64 : nullptr;
     PairTab *dt = (PairTab *)ws_get(ctx, "pairtab", sizeof(PairTab), &rc);
     if (rc) return fail(rc);
-    if ((rc = run_nodes(ctx, kind, precision, probe_q, np, step, dt, full32, o64, true))) {
+    const float cut = (float)(hipotcut_kJ / 4.184);  // mapmaker.F90:562, Real(cutoff,RSgl)
+    if ((rc = run_nodes(ctx, kind, precision, probe_q, np, step, dt, full32, o64, cut, true))) {
         if (rc == MH_EHIP) set_error("mh_map_build: node kernel launch failed");
         return fail(rc);
     }
     KTimer tcomp(ctx, "compaction");
     CompactBufs cb;
-    cb.below = (uint8_t *)ws_get(ctx, "below", nodes, &rc);
-    if (rc) return fail(rc);
-    cb.owner = (int32_t *)ws_get(ctx, "owner", sizeof(int32_t) * nodes, &rc);
-    if (rc) return fail(rc);
-    cb.cnt = (int32_t *)ws_get(ctx, "cnt", sizeof(int32_t) * nodes, &rc);
-    if (rc) return fail(rc);
-    cb.base = (int32_t *)ws_get(ctx, "base", sizeof(int32_t) * nodes, &rc);
-    if (rc) return fail(rc);
-    cb.tallies = (unsigned long long *)ws_get(ctx, "tallies", 64, &rc);
-    if (rc) return fail(rc);
-    cb.partial = (unsigned long long *)ws_get(ctx, "cpartial",
-                                              sizeof(unsigned long long) * 3 * ((nodes + 255) / 256), &rc);
-    if (rc) return fail(rc);
+    {
+        const size_t words = (size_t)compact_words(np), nb = (words + 255) / 256;
+        size_t level[4], total = al256(8 * words) + 2 * al256(40 * words) + 2 * al256(4 * words) + al256(24 * nb) + 256;
+        for (size_t l = 0, m = words; l < 4; l++) {
+            m = (m + SCAN_B - 1) / SCAN_B;
+            level[l] = al256(sizeof(int32_t) * (m + 1));
+            total += 2 * level[l];
+        }
+        char *w = (char *)ws_get(ctx, "compact", total, &rc);
+        if (rc) return fail(rc);
+        auto take = [&](size_t bytes) {
+            char *p = w;
+            w += al256(bytes);
+            return p;
+        };
+        cb.below = (u64 *)take(8 * words);
+        cb.own = (u64 *)take(40 * words);
+        cb.num = (u64 *)take(40 * words);
+        cb.cnt = (int32_t *)take(4 * words);
+        cb.base = (int32_t *)take(4 * words);
+        cb.partial = (u64 *)take(24 * nb);
+        cb.tallies = (u64 *)take(64);
+        for (int l = 0; l < 4; l++) {
+            cb.bsum[l] = (int32_t *)take(level[l]);
+            cb.boff[l] = (int32_t *)take(level[l]);
+        }
+    }
     if ((rc = map->ptr.alloc(sizeof(int32_t) * nodes))) return fail(rc);
-    const float cut = (float)(hipotcut_kJ / 4.184);  // mapmaker.F90:562, Real(cutoff,RSgl)
     int64_t total = 0;
-    if ((rc = compact_count(ctx, np, nodes, full32, cut, cb, nullptr, nullptr, map->ptr.as<int32_t>(), &total)))
+    if ((rc = compact_count(ctx, np, full32, cut, cb, &total)))
         return fail(rc);
     MH_CHECK(total < (1LL << 31), MH_ECAPACITY, "mh_map_build: more than 2^31 tabulated points");
     map->nfsize = total;
     if ((rc = map->vals.alloc(sizeof(float) * 8 * (total + 1)))) return fail(rc);
-    if ((rc = compact_assign(ctx, np, nodes, full32, cb, map->ptr.as<int32_t>(), map->vals.as<float>(), total,
-                             map->counts)))
+    if ((rc = compact_assign(ctx, np, full32, cb, map->ptr.as<int32_t>(), map->vals.as<float>(), total, map->counts)))
         return fail(rc);
     tcomp.stop();
     if (keep_full) {
@@ -1486,7 +1609,7 @@ extern "C" int mh_map_build(mh_ctx *ctx, int kind, int precision, double probe_q
 // the caller's device buffers take the compacted map, the node values and
 // compaction arrays live in the file-scope scratch array (kStaticMaxNodes
 // grid nodes at most).  No hipMalloc / hipFree / allocating library call;
-// counters and ptr are cleared by fill kernels.  Calls on one device share
+// the kernels write every counter and every ptr entry.  Calls on one device share
 // the scratch, so calls that overlap on one device race.
 extern "C" int mh_map_build_static(mh_ctx *ctx, int kind, int precision, double gridspace, double hipotcut_kJ,
                                    int32_t *ptr_dev, float *vals_dev, int64_t vals_capacity, int npnts_out[3],
@@ -1520,28 +1643,28 @@ extern "C" int mh_map_build_static(mh_ctx *ctx, int kind, int precision, double 
     MH_CHECK(sc, MH_ESTATE, "mh_map_build_static: no scratch address for this device (mh_ctx_create sets it)");
     float *full32 = (float *)(sc + kOffFull32);
     CompactBufs cb;
-    cb.below = (uint8_t *)(sc + kOffBelow);
-    cb.owner = (int32_t *)(sc + kOffOwner);
+    cb.below = (u64 *)(sc + kOffBelow);
+    cb.own = (u64 *)(sc + kOffOwn);
+    cb.num = (u64 *)(sc + kOffNum);
     cb.cnt = (int32_t *)(sc + kOffCnt);
     cb.base = (int32_t *)(sc + kOffBase);
-    cb.partial = (unsigned long long *)(sc + kOffPartial);
-    cb.tallies = (unsigned long long *)(sc + kOffTallies);
-    int32_t *bsum[4], *boff[4];
+    cb.partial = (u64 *)(sc + kOffPartial);
+    cb.tallies = (u64 *)(sc + kOffTallies);
     for (int l = 0; l < 4; l++) {
-        bsum[l] = (int32_t *)(sc + kOffScan + (2 * l) * kScanLevelBytes);
-        boff[l] = (int32_t *)(sc + kOffScan + (2 * l + 1) * kScanLevelBytes);
+        cb.bsum[l] = (int32_t *)(sc + kOffScan + (2 * l) * kScanLevelBytes);
+        cb.boff[l] = (int32_t *)(sc + kOffScan + (2 * l + 1) * kScanLevelBytes);
     }
     PairTab *dt = (PairTab *)(sc + kOffPairTab);
     int rc;
-    if ((rc = run_nodes(ctx, kind, precision, 0.0, np, step, dt, full32, nullptr, false))) {
+    const float cut = (float)(hipotcut_kJ / 4.184);  // mapmaker.F90:562, Real(cutoff,RSgl)
+    if ((rc = run_nodes(ctx, kind, precision, 0.0, np, step, dt, full32, nullptr, cut, false))) {
         if (rc == MH_EHIP) set_error("mh_map_build_static: node kernel launch failed");
         return rc;
     }
-    const float cut = (float)(hipotcut_kJ / 4.184);  // mapmaker.F90:562, Real(cutoff,RSgl)
     int64_t total = 0;
-    if ((rc = compact_count(ctx, np, nodes, full32, cut, cb, bsum, boff, ptr_dev, &total))) return rc;
+    if ((rc = compact_count(ctx, np, full32, cut, cb, &total))) return rc;
     *nfsize_out = total;
     MH_CHECK(total <= vals_capacity, MH_ECAPACITY,
              "mh_map_build_static: more tabulated points than vals_capacity records (nfsize_out holds the count)");
-    return compact_assign(ctx, np, nodes, full32, cb, ptr_dev, vals_dev, total, counts_out);
+    return compact_assign(ctx, np, full32, cb, ptr_dev, vals_dev, total, counts_out);
 }

@@ -15,7 +15,7 @@
 //     below the rounding of the FP32 values stored in the map.
 // The reference differentiates erfc exactly but evaluates it with the A&S
 // 7.1.26 fit (ewald.F90:874-916): the far field is therefore carried twice,
-// with the A&S erfc (for V) and with erfc to 1e-8 (whose interpolant is
+// with the A&S erfc (for V) and with erfc to 1e-9 (whose interpolant is
 // differentiated); the derivative terms differ from the reference's by the
 // fit's 1.5e-7 / r^2 alone.
 #include <cmath>
@@ -29,7 +29,7 @@ namespace mh {
 
 constexpr int FP = 16;            // Chebyshev points per axis
 constexpr int FPV = FP * FP * FP;
-constexpr int FDEG = 9;           // degree of the erfcx fit
+constexpr int FDEG = 10;          // degree of the erfcx fit
 constexpr int FCH = 32;           // far atoms staged per pass
 constexpr double kFarZ0 = 2.4;    // (a + R0) / a
 constexpr double kEwTokcal = 332.064;   // ewald.F90:60
@@ -46,6 +46,9 @@ struct EwP {
     double rc2, r02;
     double half[3], ihalf[3];  // half edges of a tile's box and their inverses
     double xk[FP];       // Chebyshev points on [-1, 1]
+    // bricks with a node near the compaction's cutoff
+    float cut, win;
+    int bdim[3], *blist, *bflag;
     double tc, ith;      // erfcx fit variable (t - tc) * ith
     double fit[FDEG + 1];
 };
@@ -76,6 +79,11 @@ __device__ __forceinline__ double ew_fold(double d, double L) {
     if (d > h) d = d - L;
     else if (d < -h) d = d + L;
     return d;
+}
+
+__global__ void k_ew_zero(int n, int *__restrict__ v) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) v[i] = 0;
 }
 
 // near (front, count[2 t]) and far (back, count[2 t + 1]) atoms of each tile,
@@ -457,6 +465,11 @@ __global__ void __launch_bounds__(256, 3) k_ew_nodes(EwP p, const double *__rest
                     o[2 * k + 1] = (S[i][2 * k + 1] + r.y) * kEwTokcal;
                 }
             }
+            if (FAR && fabsf((float)o[0] - p.cut) <= p.win) {
+                const int nbx = (p.n[0] + p.bdim[0] - 1) / p.bdim[0], nby = (p.n[1] + p.bdim[1] - 1) / p.bdim[1];
+                const int b = x / p.bdim[0] + nbx * (y / p.bdim[1] + nby * (z / p.bdim[2]));
+                if (atomicExch(p.bflag + b, 1) == 0) p.blist[1 + atomicAdd(p.blist, 1)] = b;
+            }
             float4 *d32 = reinterpret_cast<float4 *>(out32 + 8 * s);
             d32[0] = make_float4((float)o[0], (float)o[1], (float)o[2], (float)o[3]);
             d32[1] = make_float4((float)o[4], (float)o[5], (float)o[6], (float)o[7]);
@@ -489,7 +502,7 @@ static double erfcx_host(double x) {
 }
 
 // fit of erfcx over [x0, x1] in the variable of the A&S t; false where it
-// misses 1e-8 (a range too wide for the degree)
+// misses 1e-9 (a range too wide for the degree)
 static bool fit_erfcx(double x0, double x1, EwP &p) {
     const double pp = (double)0.3275911f;
     const double ta = 1.0 / (1.0 + pp * x1), tb = 1.0 / (1.0 + pp * x0);
@@ -517,7 +530,7 @@ static bool fit_erfcx(double x0, double x1, EwP &p) {
         const double u = -1.0 + k / 32.0, ex = erfcx_host(at(u));
         double h = p.fit[FDEG];
         for (int i = FDEG - 1; i >= 0; i--) h = h * u + p.fit[i];
-        if (!(std::fabs(h - ex) <= 1e-8 * ex)) return false;
+        if (!(std::fabs(h - ex) <= 1e-9 * ex)) return false;
     }
     return true;
 }
@@ -603,9 +616,11 @@ static void set_tiles(EwP &p, int SB) {
 // Real-space sums of every node of an orthorhombic cell plus the reciprocal
 // table: FP64 maps directly, FP32 maps (rc_real > 0) by near pairs and the
 // far field.  *done = false (and nothing launched) where the FP32 pair
-// kernel is the better route.
+// kernel is the better route.  Which nodes a map holds must not depend on
+// the route: bricks with a node near the cutoff are listed in cb and take
+// the FP32 pair kernel's values (some 70 of 150000 bricks at 334^3 nodes).
 int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], const double step[3],
-                const double *recip, float *full32, double *o64, bool *done) {
+                const double *recip, float *full32, double *o64, CutBricks &cb, bool *done) {
     EwP p;
     std::memset(&p, 0, sizeof p);
     *done = false;
@@ -697,6 +712,15 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
     if (rc) return rc;
     double *dM = (double *)ws_get(ctx, "ewcheb", sizeof(double) * M.size(), &rc);
     if (rc) return rc;
+    // number, flags, list
+    int *bl = (int *)ws_get(ctx, "ewbricks", sizeof(int) * (2 * (size_t)cb.nbricks + 2), &rc);
+    if (rc) return rc;
+    p.blist = bl + cb.nbricks;
+    p.bflag = bl;
+    p.cut = cb.cut;
+    p.win = cb.win;
+    for (int d = 0; d < 3; d++) p.bdim[d] = cb.b[d];
+    cb.list = p.blist;
     MH_HIP(hipMemcpyAsync(dM, M.data(), sizeof(double) * M.size(), hipMemcpyHostToDevice, st));
     int *plist = two ? list + tiles * p.natoms : nullptr, *pcount = two ? count + 2 * tiles : nullptr;
     double *PF = F + (size_t)2 * FPV * tiles * p.nsplit;
@@ -716,6 +740,7 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
                            ptiles, PF, dM + (size_t)2 * SB * FP, F);
     MH_HIP(hipGetLastError());
     const int nb = SB / 8;
+    hipLaunchKernelGGL(k_ew_zero, dim3((unsigned)((cb.nbricks + 256) / 256)), dim3(256), 0, st, cb.nbricks + 1, bl);
     hipLaunchKernelGGL((k_ew_nodes<4, true>), dim3((unsigned)(tiles * nb * nb)), dim3(256), 0, st, p, xyz, q, list,
                        count, F, dM, recip, full32, o64);
     MH_HIP(hipGetLastError());
