@@ -897,7 +897,6 @@ __global__ void __launch_bounds__(256) k_recip_xy(int side, int nx, int ny, int 
 //   below      nodes under the cutoff
 //   own[5]     bit planes of each node's code: the direction of its owner,
 //              (di + 1) 9 + (dj + 1) 3 + (dk + 1); 13 = none (or below)
-//   num[5]     bit planes of the number of neighbours each node owns
 //   cnt, base  indices its nodes take, their exclusive prefix sum
 // One lane per node over byte and int32 arrays (26 neighbour loads in three
 // kernels) took 2.9 ms of the 334^3 charged map.  Bound by HBM: V of every
@@ -1021,43 +1020,31 @@ __device__ __forceinline__ u64 owned_mask(const u64 *__restrict__ own, long long
     return w == 0 ? (c << 1) | ((eq(W - 1) >> lb) & 1ull) : (c << 1) | (eq(w - 1) >> 63);
 }
 
-// owned neighbours of the 64 nodes of a word (bit-sliced sums) and the
-// indices they take, one lane per word
+// indices the nodes of a word take (their own and their owned neighbours'),
+// one wave per word, lane d < 27 the mask of direction d
 __global__ void __launch_bounds__(256) k_count(int nx, int ny, int nz, int W, long long words,
                                                const u64 *__restrict__ below, const u64 *__restrict__ own,
-                                               u64 *__restrict__ num, int32_t *__restrict__ cnt) {
-    const long long word = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+                                               int32_t *__restrict__ cnt) {
+    const long long word = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
     if (word >= words) return;
     const int row = (int)(word / W), w = (int)(word - (long long)row * W);
     const int i = row / ny, j = row - i * ny;
     const u64 me = below[word];
-    u64 n[5] = {0, 0, 0, 0, 0};
+    int n = 0;
     if (me) {
-        for (int d = 0; d < 27; d++) {
-            if (d == kSelf) continue;
-            u64 c = owned_mask(own, words, nx, ny, nz, W, i, j, w, d) & me;
-#pragma unroll
-            for (int q = 0; q < 5; q++) {
-                const u64 t = n[q] & c;
-                n[q] ^= c;
-                c = t;
-            }
-        }
+        // lane kSelf counts the nodes themselves
+        if (lane < 27) n = __popcll(lane == kSelf ? me : me & owned_mask(own, words, nx, ny, nz, W, i, j, w, lane));
+        for (int o = 16; o > 0; o >>= 1) n += __shfl_xor(n, o);
     }
-    int total = __popcll(me);
-#pragma unroll
-    for (int q = 0; q < 5; q++) {
-        num[q * words + word] = n[q];
-        total += __popcll(n[q]) << q;
-    }
-    cnt[word] = total;
+    if (lane == 0) cnt[word] = n;
 }
 
 // numbers and records of a word's nodes and of the neighbours they own, one
 // wave per word (a lane per node; lane d < 27 forms the mask of direction d)
 __global__ void __launch_bounds__(256) k_assign(int nx, int ny, int nz, int W, long long words,
                                                 const u64 *__restrict__ below, const u64 *__restrict__ own,
-                                                const u64 *__restrict__ num, const int32_t *__restrict__ base,
+                                                const int32_t *__restrict__ base,
                                                 const float *__restrict__ full, int32_t *__restrict__ ptr,
                                                 float *__restrict__ cvals) {
     const long long word = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1073,15 +1060,21 @@ __global__ void __launch_bounds__(256) k_assign(int nx, int ny, int nz, int W, l
         return (u64)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)mask, d) |
                ((u64)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(mask >> 32), d) << 32);
     };
-    auto lower = [&](u64 m) {  // bits of m below the lane's
-        return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-    };
     const bool mine = (me >> lane) & 1ull;
     if (z < nz && !mine && ((of(kSelf) >> lane) & 1ull)) ptr[(long long)row * nz + z] = 0;
     if (!me) return;
-    long long idx = (long long)base[word] + lower(me);
-#pragma unroll
-    for (int q = 0; q < 5; q++) idx += (long long)lower(num[q * words + word]) << q;
+    // indices the lane's node takes, and those of the lanes below it
+    int n = 0;
+    for (int d = 0; d < 27; d++) {
+        const u64 m = d == kSelf ? me : of(d);
+        n += (int)((m >> lane) & 1ull);
+    }
+    int incl = n;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl, o);
+        if (lane >= o) incl += v;
+    }
+    long long idx = (long long)base[word] + incl - n;
     auto put = [&](long long t, long long k) {
         ptr[t] = (int32_t)(k + 1);
         const float4 *src = reinterpret_cast<const float4 *>(full + 8 * t);
@@ -1156,8 +1149,7 @@ constexpr long long kStaticScan0 = kStaticMaxWords / 1024 + 2;
 constexpr size_t kOffFull32 = 0;
 constexpr size_t kOffBelow = kOffFull32 + al256(sizeof(float) * 8 * kStaticMaxNodes);
 constexpr size_t kOffOwn = kOffBelow + al256(sizeof(u64) * kStaticMaxWords);
-constexpr size_t kOffNum = kOffOwn + al256(sizeof(u64) * 5 * kStaticMaxWords);
-constexpr size_t kOffCnt = kOffNum + al256(sizeof(u64) * 5 * kStaticMaxWords);
+constexpr size_t kOffCnt = kOffOwn + al256(sizeof(u64) * 5 * kStaticMaxWords);
 constexpr size_t kOffBase = kOffCnt + al256(sizeof(int32_t) * kStaticMaxWords);
 constexpr size_t kOffPartial = kOffBase + al256(sizeof(int32_t) * kStaticMaxWords);
 constexpr size_t kOffTallies = kOffPartial + al256(sizeof(u64) * 3 * kStaticBlocks256);
@@ -1225,7 +1217,7 @@ static int scan_exclusive_b(mh_ctx *ctx, int level, long long n, const int32_t *
 
 // compaction buffers (pmap_compact restated for the device)
 struct CompactBufs {
-    u64 *below, *own, *num;
+    u64 *below, *own;
     int32_t *cnt, *base;
     u64 *tallies, *partial;
     int32_t *bsum[4], *boff[4];  // levels of the prefix sum
@@ -1244,8 +1236,7 @@ static int compact_count(mh_ctx *ctx, const int np[3], const float *full32, floa
     const unsigned gw = (unsigned)((words + 255) / 256), gq = (unsigned)((words + 3) / 4);
     hipLaunchKernelGGL(k_below, dim3(gq), dim3(256), 0, st, np[0] * np[1], np[2], W, full32, cut, b.below);
     hipLaunchKernelGGL(k_owner, dim3(gw), dim3(256), 0, st, np[0], np[1], np[2], W, words, b.below, b.own, b.partial);
-    hipLaunchKernelGGL(k_count, dim3(gw), dim3(256), 0, st, np[0], np[1], np[2], W, words, b.below, b.own, b.num,
-                       b.cnt);
+    hipLaunchKernelGGL(k_count, dim3(gq), dim3(256), 0, st, np[0], np[1], np[2], W, words, b.below, b.own, b.cnt);
     hipLaunchKernelGGL(k_tally, dim3(1), dim3(1024), 0, st, (long long)gw, b.partial, b.tallies);
     if (hipGetLastError() != hipSuccess) {
         set_error("map compaction: kernel launch failed");
@@ -1261,7 +1252,7 @@ static int compact_assign(mh_ctx *ctx, const int np[3], const float *full32, con
     const int W = (np[2] + 63) / 64;
     const long long words = compact_words(np);
     hipLaunchKernelGGL(k_assign, dim3((unsigned)((words + 3) / 4)), dim3(256), 0, st, np[0], np[1], np[2], W, words,
-                       b.below, b.own, b.num, b.base, full32, ptr, vals);
+                       b.below, b.own, b.base, full32, ptr, vals);
     if (hipGetLastError() != hipSuccess) {
         set_error("map compaction: assign kernel launch failed");
         return MH_EHIP;
@@ -1556,7 +1547,7 @@ extern "C" int mh_map_build(mh_ctx *ctx, int kind, int precision, double probe_q
     CompactBufs cb;
     {
         const size_t words = (size_t)compact_words(np), nb = (words + 255) / 256;
-        size_t level[4], total = al256(8 * words) + 2 * al256(40 * words) + 2 * al256(4 * words) + al256(24 * nb) + 256;
+        size_t level[4], total = al256(8 * words) + al256(40 * words) + 2 * al256(4 * words) + al256(24 * nb) + 256;
         for (size_t l = 0, m = words; l < 4; l++) {
             m = (m + SCAN_B - 1) / SCAN_B;
             level[l] = al256(sizeof(int32_t) * (m + 1));
@@ -1571,7 +1562,6 @@ extern "C" int mh_map_build(mh_ctx *ctx, int kind, int precision, double probe_q
         };
         cb.below = (u64 *)take(8 * words);
         cb.own = (u64 *)take(40 * words);
-        cb.num = (u64 *)take(40 * words);
         cb.cnt = (int32_t *)take(4 * words);
         cb.base = (int32_t *)take(4 * words);
         cb.partial = (u64 *)take(24 * nb);
@@ -1645,7 +1635,6 @@ extern "C" int mh_map_build_static(mh_ctx *ctx, int kind, int precision, double 
     CompactBufs cb;
     cb.below = (u64 *)(sc + kOffBelow);
     cb.own = (u64 *)(sc + kOffOwn);
-    cb.num = (u64 *)(sc + kOffNum);
     cb.cnt = (int32_t *)(sc + kOffCnt);
     cb.base = (int32_t *)(sc + kOffBase);
     cb.partial = (u64 *)(sc + kOffPartial);
