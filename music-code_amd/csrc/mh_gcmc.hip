@@ -26,6 +26,7 @@
 //   scalars: N, energy, sumN, sumN2, nsteps, att[4], acc[4], rng ix/iy/first/iseed
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "mh_device.h"
@@ -509,7 +510,7 @@ __device__ __forceinline__ double2 k_delta(const GDev &P, const Shared &sh, int 
 // Energy terms of a move: set A (+) and set B (-) of one molecule of species
 // sh.spc against every other molecule of every species (skip = its slot in
 // its species, N = that species' count) and the reciprocal-space delta,
-// whose dS(k) is left in K.d (registers) or dSg (KPL == 0).
+// whose dS(k) is left in K.d (registers) or dSg (KPL == 0; NULL: not kept).
 // out: map A, pairs A, map B, pairs B, reciprocal delta, ok(A).
 // Centre-of-mass cutoffs (P.comcut): ctrg = the replica's molecule centres
 // [slots][3]; set A's centre is cA (a stored molecule) or the mean of
@@ -783,7 +784,7 @@ __device__ __forceinline__ void move_energy(const GDev &P, Shared &sh, const dou
                 const double2 s = Sg[k];
                 const double nre = s.x + d.x, nim = s.y + d.y;
                 eK += P.wk[k] * ((nre * nre + nim * nim) - (s.x * s.x + s.y * s.y));
-                dSg[k] = d;
+                if (dSg) dSg[k] = d;
             }
         }
     }
@@ -1424,12 +1425,13 @@ __global__ void __launch_bounds__(NT) k_gcmc(const GDev *__restrict__ Ptab, Rep 
     }
 }
 
-// Insertion energies of trial molecules (one workgroup per trial)
+// Insertion energies of trial molecules (one workgroup per trial).  No trial
+// is accepted, so dS(k) stays in registers: storing it took 110 MB, allocated
+// and written per call, for 4096 trials of 1687 k vectors (3160 us a call).
 template <int NT, int PREC>
 __global__ void __launch_bounds__(NT) k_trial(const GDev *__restrict__ Ptab, Rep R, int rep, int spc, int n,
                                                const double *__restrict__ tcom, const double *__restrict__ tang,
-                                               double2 *__restrict__ dSbuf, double *__restrict__ e,
-                                               uint8_t *__restrict__ okout) {
+                                               double *__restrict__ e, uint8_t *__restrict__ okout) {
     __shared__ Shared sh;
     __shared__ GDev P;
     const int tid = threadIdx.x;
@@ -1454,11 +1456,11 @@ __global__ void __launch_bounds__(NT) k_trial(const GDev *__restrict__ Ptab, Rep
     double o[6];
     KReg<0> K;
     if (P.slanted)
-        move_energy<NT, PREC, 0, true>(P, sh, pos, N, -1, true, false, 1.0, K, S, dSbuf + (long long)t * P.nk,
-                                       nullptr, o, ctrg, nullptr, nullptr);
+        move_energy<NT, PREC, 0, true>(P, sh, pos, N, -1, true, false, 1.0, K, S, nullptr, nullptr, o, ctrg,
+                                       nullptr, nullptr);
     else
-        move_energy<NT, PREC, 0>(P, sh, pos, N, -1, true, false, 1.0, K, S, dSbuf + (long long)t * P.nk, nullptr, o,
-                                 ctrg, nullptr, nullptr);
+        move_energy<NT, PREC, 0>(P, sh, pos, N, -1, true, false, 1.0, K, S, nullptr, nullptr, o, ctrg, nullptr,
+                                 nullptr);
     if (tid == 0) {
         double U = __dadd_rn(o[0], o[1]);
         if (P.ewald) U = U + o[4] + P.molconst;
@@ -1644,6 +1646,8 @@ struct mh_gcmc {
     bool ldsmol = false;    // molecules held in LDS during a launch
     bool slanted = false;   // single system in a slanted cell
     size_t lds_bytes = 0;   // dynamic LDS of the launch
+    DBuf trial;             // buffers of mh_trial_energy
+    std::mutex trial_mu;
     bool exy_off = false;   // autotuner: e^{i(kx x + ky y)} tables disabled
     bool pool = false;      // slot pool (per-replica system and step budget)
     std::vector<SysHost> sys;
@@ -2837,28 +2841,31 @@ int mh_trial_energy(mh_gcmc *g, int rep, int n, const double *com, const double 
              "mh_trial_energy: bad arguments");
     if (n == 0) return MH_OK;
     MH_HIP(hipSetDevice(g->ctx->device));
-    DBuf dc, da, de, dok, dsb;
-    int rc;
-    if ((rc = dc.alloc(sizeof(double) * 3 * n)) || (rc = da.alloc(sizeof(double) * 3 * n)) ||
-        (rc = de.alloc(sizeof(double) * n)) || (rc = dok.alloc(n)) ||
-        (rc = dsb.alloc(sizeof(double2) * (size_t)n * (g->nk + 1))))
-        return rc;
-    std::vector<double> za(3 * (size_t)n, 0.0);
-    MH_HIP(hipMemcpy(dc.p, com, sizeof(double) * 3 * n, hipMemcpyHostToDevice));
-    MH_HIP(hipMemcpy(da.p, ang ? ang : za.data(), sizeof(double) * 3 * n, hipMemcpyHostToDevice));
+    // centres, angles, energies, flags in one buffer kept with the batch (its
+    // callers take turns)
+    const size_t c3 = sizeof(double) * 3 * n, need = 2 * c3 + (sizeof(double) + 1) * n;
+    std::lock_guard<std::mutex> lk(g->trial_mu);
+    if (g->trial.n < need)
+        if (int rc = g->trial.alloc(need)) return rc;
+    char *w = g->trial.as<char>();
+    double *dc = (double *)w, *da = dc + 3 * (size_t)n, *de = da + 3 * (size_t)n;
+    uint8_t *dok = (uint8_t *)(de + n);
+    hipStream_t st = g->ctx->stream;
+    std::vector<double> za;
+    if (!ang) za.assign(3 * (size_t)n, 0.0);
+    MH_HIP(hipMemcpyAsync(dc, com, c3, hipMemcpyHostToDevice, st));
+    MH_HIP(hipMemcpyAsync(da, ang ? ang : za.data(), c3, hipMemcpyHostToDevice, st));
     Rep r = g->rep();
     if (g->prec == MH_PREC_FP32)
-        hipLaunchKernelGGL((k_trial<256, MH_PREC_FP32>), dim3(n), dim3(256), 0, g->ctx->stream, g->dP.as<GDev>(), r,
-                           rep, g->sel, n, dc.as<double>(), da.as<double>(), dsb.as<double2>(), de.as<double>(),
-                           dok.as<uint8_t>());
+        hipLaunchKernelGGL((k_trial<256, MH_PREC_FP32>), dim3(n), dim3(256), 0, st, g->dP.as<GDev>(), r, rep, g->sel,
+                           n, dc, da, de, dok);
     else
-        hipLaunchKernelGGL((k_trial<256, MH_PREC_FP64>), dim3(n), dim3(256), 0, g->ctx->stream, g->dP.as<GDev>(), r,
-                           rep, g->sel, n, dc.as<double>(), da.as<double>(), dsb.as<double2>(), de.as<double>(),
-                           dok.as<uint8_t>());
+        hipLaunchKernelGGL((k_trial<256, MH_PREC_FP64>), dim3(n), dim3(256), 0, st, g->dP.as<GDev>(), r, rep, g->sel,
+                           n, dc, da, de, dok);
     MH_HIP(hipGetLastError());
-    MH_HIP(hipStreamSynchronize(g->ctx->stream));
-    MH_HIP(hipMemcpy(e, de.p, sizeof(double) * n, hipMemcpyDeviceToHost));
-    MH_HIP(hipMemcpy(ok, dok.p, n, hipMemcpyDeviceToHost));
+    MH_HIP(hipMemcpyAsync(e, de, sizeof(double) * n, hipMemcpyDeviceToHost, st));
+    MH_HIP(hipMemcpyAsync(ok, dok, n, hipMemcpyDeviceToHost, st));
+    MH_HIP(hipStreamSynchronize(st));
     return MH_OK;
 }
 
