@@ -25,6 +25,8 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "mh_device.h"
@@ -35,6 +37,7 @@ namespace mh {
 
 constexpr int HS = MH_MAX_SITES;
 constexpr int HT = 16;
+constexpr int kQuad = 4;   // lanes that share a site's map and LJ terms
 constexpr int JLEV = 20;  // jump-ahead levels: up to 2^20 draws per move
 // neighbour lists: partner sites within hicut + kSkin, rebuilt whenever a
 // site has moved more than half the skin since the last build (pairs left out
@@ -78,6 +81,7 @@ struct HRep {
     double *v, *a;              // [rep][maxN][ns][3] velocities, accelerations
     uint16_t *nbl;              // [rep][cap][cap] neighbour lists, entry-major
     int cap;                    // maxN * nsites
+    double *fx;                 // [rep][2][cap][3] partial forces (NULL: in LDS)
 };
 
 constexpr double kScaleKE = 0.01;   // (A/ps)^2 amu -> kJ/mol, defaults.F90:76
@@ -128,119 +132,84 @@ __device__ double gauss_pair(const HDev &P, const Rng &S0, unsigned p, int secon
     return second ? rad * sin(twopi * r2) : rad * cos(twopi * r2);
 }
 
-// forcehermite (interpolate.F90:189-584) in two parts, so that other work
-// can run while the corner records are in flight.  hermite_fetch: the cell of
-// a position (false outside the tabulated range) and the loads of its eight
-// corner records (global address space, so waits on LDS reads do not wait on
-// them).
+// forcehermite (interpolate.F90:189-584) over the lanes of a quad, two cell
+// corners each, in two parts, so that other work can run while the corner
+// records are in flight.  hermite_fetch: the cell of a position (false outside
+// the tabulated range) and the loads of the lane's corner records (global
+// address space, so waits on LDS reads do not wait on them).
+constexpr int QC = 8 / kQuad;  // corners per lane
 struct Corners {
-    float4 rec[16];
+    float4 rec[2 * QC];
     double t[3];
 };
 
 typedef float F4v __attribute__((ext_vector_type(4)));
 typedef const F4v __attribute__((address_space(1))) *GlobalF4;
 
-__device__ __forceinline__ bool hermite_fetch(const MapRef &m, const double *r, Corners &g) {
+__device__ __forceinline__ bool hermite_fetch(const MapRef &m, const double *r, int l, Corners &g) {
     int i0[3], i1[3];
     for (int d = 0; d < 3; d++)
         if (!cell_axis(r[d], m.ell[d], m.step[d], m.n[d], i0[d], i1[d], g.t[d])) return false;
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const int cx = (kCX >> c) & 1, cy = (kCY >> c) & 1, cz = (kCZ >> c) & 1;
+    for (int k = 0; k < QC; k++) {
+        const int c = l * QC + k, cx = (kCX >> c) & 1, cy = (kCY >> c) & 1, cz = (kCZ >> c) & 1;
         const long long node = ((long long)(cx ? i1[0] : i0[0]) * m.n[1] + (cy ? i1[1] : i0[1])) * m.n[2] +
                                (cz ? i1[2] : i0[2]);
         const GlobalF4 q = (GlobalF4)(m.dense + 8 * node);
         const F4v lo = q[0], hi = q[1];
-        g.rec[2 * c] = make_float4(lo.x, lo.y, lo.z, lo.w);
-        g.rec[2 * c + 1] = make_float4(hi.x, hi.y, hi.z, hi.w);
+        g.rec[2 * k] = make_float4(lo.x, lo.y, lo.z, lo.w);
+        g.rec[2 * k + 1] = make_float4(hi.x, hi.y, hi.z, hi.w);
     }
     return true;
 }
 
-// hermite_eval: p = V, -dV/dx, -dV/dy, -dV/dz from the fetched corners;
-// false where a corner is untabulated
+// hermite_eval: the lane's share of p = V, -dV/dx, -dV/dy, -dV/dz; false
+// where one of its corners is untabulated
 template <int PREC>
-__device__ __forceinline__ bool hermite_eval(const MapRef &m, const Corners &g, double p[4]) {
+__device__ __forceinline__ bool hermite_eval(const MapRef &m, const Corners &g, int l, double p[4]) {
     bool ok = true;
 #pragma unroll
-    for (int c = 0; c < 8; c++) ok = ok && g.rec[2 * c].x == g.rec[2 * c].x;
+    for (int k = 0; k < QC; k++) ok = ok && g.rec[2 * k].x == g.rec[2 * k].x;
     if (!ok) return false;
-    if (PREC == MH_PREC_FP64) {
-        double h[3][2][2], hd[3][2][2];
-        for (int d = 0; d < 3; d++) {
-            const double st = m.step[d], u = g.t[d], w = 1 - g.t[d];
-            h[d][0][0] = w * w * (3.0 - 2.0 * w);
-            h[d][1][0] = u * u * (3.0 - 2.0 * u);
-            h[d][0][1] = (-st) * w * w * (w - 1.0);
-            h[d][1][1] = st * u * u * (u - 1.0);
-            hd[d][0][0] = -(6.0 * w * (1.0 - w));
-            hd[d][1][0] = 6.0 * u * (1.0 - u);
-            hd[d][0][1] = -((-st) * w * (3.0 * w - 2.0));
-            hd[d][1][1] = st * u * (3.0 * u - 2.0);
-        }
-        double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
+    using T = typename std::conditional<PREC == MH_PREC_FP64, double, float>::type;
+    double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const int cx = (kCX >> c) & 1, cy = (kCY >> c) & 1, cz = (kCZ >> c) & 1;
-            const float4 a = g.rec[2 * c], b = g.rec[2 * c + 1];
-            const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const int dx = (kCX >> k) & 1, dy = (kCY >> k) & 1, dz = (kCZ >> k) & 1;
-                const double fv = f[k], hi = h[0][cx][dx], hj = h[1][cy][dy], hk = h[2][cz][dz];
-                const double di = hd[0][cx][dx], dj = hd[1][cy][dy], dk = hd[2][cz][dz];
-                s1 = s1 + fv * hi * hj * hk;
-                s2 = s2 + fv * di * hj * hk;
-                s3 = s3 + fv * hi * dj * hk;
-                s4 = s4 + fv * hi * hj * dk;
-            }
-        }
-        p[0] = s1;
-        p[1] = -s2 / m.step[0];
-        p[2] = -s3 / m.step[1];
-        p[3] = -s4 / m.step[2];
-    } else {
+    for (int kc = 0; kc < QC; kc++) {
 #pragma clang fp contract(fast)
-        float h[3][2][2], hd[3][2][2];
+        const int c = l * QC + kc;
+        const int up[3] = {(kCX >> c) & 1, (kCY >> c) & 1, (kCZ >> c) & 1};
+        // the corner's two basis functions per axis (value, slope) and their derivatives
+        T h[3][2], hd[3][2];
         for (int d = 0; d < 3; d++) {
-            const float st = (float)m.step[d], u = (float)g.t[d], w = 1.0f - u;
-            h[d][0][0] = w * w * (3.0f - 2.0f * w);
-            h[d][1][0] = u * u * (3.0f - 2.0f * u);
-            h[d][0][1] = (-st) * w * w * (w - 1.0f);
-            h[d][1][1] = st * u * u * (u - 1.0f);
-            hd[d][0][0] = -(6.0f * w * (1.0f - w));
-            hd[d][1][0] = 6.0f * u * (1.0f - u);
-            hd[d][0][1] = -((-st) * w * (3.0f * w - 2.0f));
-            hd[d][1][1] = st * u * (3.0f * u - 2.0f);
+            const T st = (T)m.step[d], u = up[d] ? (T)g.t[d] : (T)1 - (T)g.t[d];
+            const T ss = up[d] ? st : -st;
+            h[d][0] = u * u * ((T)3 - (T)2 * u);
+            h[d][1] = ss * u * u * (u - (T)1);
+            const T d0 = (T)6 * u * ((T)1 - u), d1 = ss * u * ((T)3 * u - (T)2);
+            hd[d][0] = up[d] ? d0 : -d0;
+            hd[d][1] = up[d] ? d1 : -d1;
         }
-        double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
+        const float4 a = g.rec[2 * kc], b = g.rec[2 * kc + 1];
+        const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        T q1 = 0, q2 = 0, q3 = 0, q4 = 0;
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const int cx = (kCX >> c) & 1, cy = (kCY >> c) & 1, cz = (kCZ >> c) & 1;
-            const float4 a = g.rec[2 * c], b = g.rec[2 * c + 1];
-            const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-            float q1 = 0.0f, q2 = 0.0f, q3 = 0.0f, q4 = 0.0f;
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const int dx = (kCX >> k) & 1, dy = (kCY >> k) & 1, dz = (kCZ >> k) & 1;
-                const float hi = h[0][cx][dx], hj = h[1][cy][dy], hk = h[2][cz][dz];
-                const float di = hd[0][cx][dx], dj = hd[1][cy][dy], dk = hd[2][cz][dz];
-                q1 += f[k] * hi * hj * hk;
-                q2 += f[k] * di * hj * hk;
-                q3 += f[k] * hi * dj * hk;
-                q4 += f[k] * hi * hj * dk;
-            }
-            s1 += q1;
-            s2 += q2;
-            s3 += q3;
-            s4 += q4;
+        for (int k = 0; k < 8; k++) {
+            const int dx = (kCX >> k) & 1, dy = (kCY >> k) & 1, dz = (kCZ >> k) & 1;
+            const T fv = f[k], hi = h[0][dx], hj = h[1][dy], hk = h[2][dz];
+            q1 += fv * hi * hj * hk;
+            q2 += fv * hd[0][dx] * hj * hk;
+            q3 += fv * hi * hd[1][dy] * hk;
+            q4 += fv * hi * hj * hd[2][dz];
         }
-        p[0] = s1;
-        p[1] = -s2 / m.step[0];
-        p[2] = -s3 / m.step[1];
-        p[3] = -s4 / m.step[2];
+        s1 += (double)q1;
+        s2 += (double)q2;
+        s3 += (double)q3;
+        s4 += (double)q4;
     }
+    p[0] = s1;
+    p[1] = -s2 / m.step[0];
+    p[2] = -s3 / m.step[1];
+    p[3] = -s4 / m.step[2];
     return true;
 }
 
@@ -250,9 +219,10 @@ __device__ __forceinline__ double dot3(const double *a, const double *b) {
 
 // bonded terms containing atom `a` of molecule R (principal coordinates):
 // force on a into f, energy of terms whose first atom is a into eb (stretch,
-// bending, torsion)
-__device__ void bonded_site(const HDev &P, const double *R, int a, double f[3], double (&eb)[3]) {
-    for (int q = 0; q < P.nb; q++) {  // harmonic_getinteraction, harmonic.F90:130-160
+// bending, torsion); every stride-th term of a kind from `first` on
+__device__ void bonded_site(const HDev &P, const double *R, int a, double f[3], double (&eb)[3], int first = 0,
+                            int stride = 1) {
+    for (int q = first; q < P.nb; q += stride) {  // harmonic_getinteraction, harmonic.F90:130-160
         const int i = P.bi[q][0], j = P.bi[q][1];
         if (a != i && a != j) continue;
         double vr[3] = {R[3 * j] - R[3 * i], R[3 * j + 1] - R[3 * i + 1], R[3 * j + 2] - R[3 * i + 2]};
@@ -265,7 +235,7 @@ __device__ void bonded_site(const HDev &P, const double *R, int a, double f[3], 
         for (int k = 0; k < 3; k++) f[k] += (a == j) ? vru[k] * fm : vru[k] * fm * (-1.0);
         if (a == i) eb[0] += 0.5 * k_ * (r - req) * (r - req);
     }
-    for (int q = 0; q < P.na; q++) {  // harmonica, harmonica.F90:100-160
+    for (int q = first; q < P.na; q += stride) {  // harmonica, harmonica.F90:100-160
         const int i = P.ai[q][0], j = P.ai[q][1], l = P.ai[q][2];
         if (a != i && a != j && a != l) continue;
         double v1[3], v2[3];
@@ -287,7 +257,7 @@ __device__ void bonded_site(const HDev &P, const double *R, int a, double f[3], 
         }
         if (a == i) eb[1] += 0.5 * P.ak[q] * (th - P.at0[q]) * (th - P.at0[q]);
     }
-    for (int q = 0; q < P.nt; q++) {  // cosexpansion_getinteraction, cosexpansion.F90:88-196
+    for (int q = first; q < P.nt; q += stride) {  // cosexpansion_getinteraction, cosexpansion.F90:88-196
         const int i1 = P.ti[q][0], i2 = P.ti[q][1], i3 = P.ti[q][2], i4 = P.ti[q][3];
         if (a != i1 && a != i2 && a != i3 && a != i4) continue;
         double va[3], vb[3], vc[3];
@@ -332,10 +302,13 @@ __device__ void bonded_site(const HDev &P, const double *R, int a, double f[3], 
 // fixed-point cell position of site s (x 2^32 / L, wrapped mod 2^32: the
 // difference of two such coordinates read as int32 is the minimum image) and
 // its atom index a
-__device__ __forceinline__ void put_fx(const HDev &P, uint4 *ru, const double *r, int s, int a) {
+__device__ __forceinline__ uint4 fx_of(const HDev &P, const double *r, int a) {
     uint32_t u[3];
-    for (int d = 0; d < 3; d++) u[d] = (uint32_t)(unsigned long long)(long long)rint(r[3 * s + d] * P.fxs[d]);
-    ru[s] = make_uint4(u[0], u[1], u[2], (uint32_t)a);
+    for (int d = 0; d < 3; d++) u[d] = (uint32_t)(unsigned long long)(long long)rint(r[d] * P.fxs[d]);
+    return make_uint4(u[0], u[1], u[2], (uint32_t)a);
+}
+__device__ __forceinline__ void put_fx(const HDev &P, uint4 *ru, const double *r, int s, int a) {
+    ru[s] = fx_of(P, r + 3 * s, a);
 }
 
 // true where one of the lane's sites has moved more than half the skin (in
@@ -381,152 +354,203 @@ __device__ void hmc_lists(const HDev &P, const uint4 *ru, const double *rp, int 
         }
         nb[s] = make_float4((float)rp[3 * s], (float)rp[3 * s + 1], (float)rp[3 * s + 2], __int_as_float(c));
     }
+    __syncthreads();  // other lanes read the lists
 }
 
-// f(j) for the entries of a neighbour list in order; the next group of eight
-// entries is loaded while a group is processed
+// f(j) for every kQuad-th entry of a neighbour list from entry l on; the next
+// group of four entries is loaded while a group is processed
 template <class Fn>
-__device__ __forceinline__ void list_loop(const uint16_t *nbl, unsigned s, int n, unsigned cap, Fn &&f) {
-    int q = 0;
-    unsigned o = s;  // offset of entry q
-    if (n >= 8) {
-        int cur[8];
+__device__ __forceinline__ void list_loop(const uint16_t *nbl, unsigned s, int l, int n, unsigned cap, Fn &&f) {
+    constexpr int U = 4;
+    const unsigned st = kQuad * cap;
+    int left = (n - l + kQuad - 1) / kQuad;
+    unsigned o = s + (unsigned)l * cap;  // offset of the next entry
+    if (left >= U) {
+        int cur[U];
 #pragma unroll
-        for (int u = 0; u < 8; u++) cur[u] = nbl[o + u * cap];
-        for (; q + 8 <= n; q += 8) {
-            int nxt[8];
-            const bool more = q + 16 <= n;
-            o += 8 * cap;
+        for (int u = 0; u < U; u++) cur[u] = nbl[o + u * st];
+        for (; left >= U; left -= U) {
+            int nxt[U];
+            const bool more = left >= 2 * U;
+            o += U * st;
             if (more) {
 #pragma unroll
-                for (int u = 0; u < 8; u++) nxt[u] = nbl[o + u * cap];
+                for (int u = 0; u < U; u++) nxt[u] = nbl[o + u * st];
             }
 #pragma unroll
-            for (int u = 0; u < 8; u++) f(cur[u]);
+            for (int u = 0; u < U; u++) f(cur[u]);
             if (more) {
 #pragma unroll
-                for (int u = 0; u < 8; u++) cur[u] = nxt[u];
+                for (int u = 0; u < U; u++) cur[u] = nxt[u];
             }
         }
     }
-    for (; q < n; q++, o += cap) f(nbl[o]);
+    for (; left > 0; left--, o += st) f(nbl[o]);
 }
 
 // energy parts of a configuration: framework map, sorbate-sorbate LJ,
 // stretch, bending, torsion
 constexpr int kParts = 5;
 
-// force on site s (map, sorbate-sorbate LJ over its neighbour list, bonded
-// terms) into f; its energy shares added to ep; bad on a failed evaluation
+// minimum image without branches: d - L rint(d / L), the same value as the
+// single fold but for d at exactly half an edge
+__device__ __forceinline__ double fold_rint(double d, double L, double iL) { return fma(-L, rint(d * iL), d); }
+
+// one LJ pair of site s: FP64 from the positions, FP32 from the fixed-point
+// copies; energy and force added to el, f
 template <int PREC>
-__device__ __forceinline__ void site_force(const HDev &P, const double *rp, const double *r, const uint4 *ru,
-                                           const uint16_t *nbl, int cap, int s, int n, double f[3],
-                                           double (&ep)[kParts], double &bad) {
-    const int ns = P.ns, m = s / ns, a = s - m * ns;
+struct PairSum {
+    double el = 0.0, f[3] = {0.0, 0.0, 0.0};
+    float elf = 0.0f, ff[3] = {0.0f, 0.0f, 0.0f};
+    bool bad = false;
+    double iL[3];
+    __device__ __forceinline__ PairSum(const HDev &P) {
+        for (int d = 0; d < 3; d++) iL[d] = PREC == MH_PREC_FP64 ? 1.0 / P.full[d] : 0.0;
+    }
+    __device__ __forceinline__ void pair64(const HDev &P, const double *pr, const double *ri, const double *rj) {
+        const double sx = fold_rint(ri[0] - rj[0], P.full[0], iL[0]);
+        const double sy = fold_rint(ri[1] - rj[1], P.full[1], iL[1]);
+        const double sz = fold_rint(ri[2] - rj[2], P.full[2], iL[2]);
+        const double r2 = fma(sx, sx, fma(sy, sy, sz * sz));
+        if (r2 > pr[2]) return;
+        if (r2 < pr[3]) bad = true;
+        // 1 / r^2: the hardware's approximation and two Newton steps
+        double r2i = __builtin_amdgcn_rcp(r2);
+        r2i = fma(r2i, fma(-r2, r2i, 1.0), r2i);
+        r2i = fma(r2i, fma(-r2, r2i, 1.0), r2i);
+        const double r6i = r2i * r2i * r2i, ta = pr[0] * (r6i * r6i), tb = pr[1] * r6i;
+        el += ta - tb;
+        const double fm = fma(12.0, ta, -6.0 * tb) * r2i;
+        f[0] = fma(sx, fm, f[0]);
+        f[1] = fma(sy, fm, f[1]);
+        f[2] = fma(sz, fm, f[2]);
+    }
+    __device__ __forceinline__ void pair32(const HDev &P, const float4 *pp, const uint4 pi, const uint4 pj) {
+#pragma clang fp contract(fast)
+        const float x = (float)(int)(pi.x - pj.x) * P.fxu[0], y = (float)(int)(pi.y - pj.y) * P.fxu[1],
+                    z = (float)(int)(pi.z - pj.z) * P.fxu[2];
+        const float r2 = x * x + y * y + z * z;
+        const float4 pr = pp[pj.w];
+        const bool in = !(r2 > pr.z);
+        bad |= in && r2 < pr.w;
+        // A/r^12 - B/r^6 and its force factor (12 A/r^12 - 6 B/r^6)/r^2
+        const float r2i = in ? rcp_fast(r2) : 0.0f, r6i = r2i * r2i * r2i;
+        const float ta = pr.x * r6i * r6i, tb = pr.y * r6i, de = ta - tb;
+        elf += de;
+        const float fm = (de + ta) * (6.0f * r2i);
+        ff[0] += x * fm;
+        ff[1] += y * fm;
+        ff[2] += z * fm;
+    }
+    // the lane's totals into FP64
+    __device__ __forceinline__ void close() {
+        if (PREC == MH_PREC_FP64) return;
+        el = elf;
+        for (int d = 0; d < 3; d++) f[d] = ff[d];
+    }
+};
+
+// the quad's sum of v, in every lane
+__device__ __forceinline__ double quad_sum(double v) {
+    v += dpp_f64<0xB1>(v);  // lanes 1 0 3 2
+    v += dpp_f64<0x4E>(v);  // lanes 2 3 0 1
+    return v;
+}
+
+// map and sorbate-sorbate LJ terms of site s, the lanes of a quad sharing
+// them (two map corners and every fourth list entry each): the force on the
+// site in every lane of the quad, its energy shares in the lanes' ep
+template <int PREC>
+__device__ __forceinline__ void site_force(const HDev &P, const double *r, const uint4 *ru, const uint16_t *nbl,
+                                           int cap, int s, int l, int n, double f[3], double (&ep)[kParts],
+                                           double &bad) {
+    const int a = s - (s / P.ns) * P.ns;
     const double *ri = r + 3 * s;
-    f[0] = f[1] = f[2] = 0.0;
-    // map corners requested first; in FP32 the bonded terms are evaluated
-    // while they arrive (in FP64 that costs more registers than it saves).
-    // The bonded terms are added last.
+    // map corners requested first, evaluated after the pairs
     Corners g;
     const bool mapped = P.has_map[a] != 0;
-    const bool inside = mapped && hermite_fetch(P.map[a], ri, g);
-    double fb[3] = {0.0, 0.0, 0.0}, eb[3] = {0.0, 0.0, 0.0};
-    if (PREC != MH_PREC_FP64) bonded_site(P, rp + 3 * (m * ns), a, fb, eb);
+    const bool inside = mapped && hermite_fetch(P.map[a], ri, l, g);
+    // LJ against the listed partners: the list holds every partner within
+    // hicut, so the sums are those of the loop over all sites of the other
+    // molecules that skips pairs beyond hicut and switched-off type pairs
+    PairSum<PREC> ps(P);
+    if (PREC == MH_PREC_FP64) {
+        const double(*pp)[4] = P.pp64 + a * HS;
+        const double rs[3] = {ri[0], ri[1], ri[2]};
+        list_loop(nbl, (unsigned)s, l, n, (unsigned)cap, [&](int j) { ps.pair64(P, pp[ru[j].w], rs, r + 3 * j); });
+    } else {
+        const uint4 pi = ru[s];
+        const float4 *pp = P.pp32 + a * HS;
+        list_loop(nbl, (unsigned)s, l, n, (unsigned)cap, [&](int j) { ps.pair32(P, pp, pi, ru[j]); });
+    }
+    ps.close();
+    if (ps.bad) bad = 1.0;
+    ep[1] += 0.5 * ps.el;  // each pair is seen from both of its sites
+    for (int d = 0; d < 3; d++) f[d] = ps.f[d];
     if (mapped) {
         double p[4];
-        if (inside && hermite_eval<PREC>(P.map[a], g, p)) {
+        if (inside && hermite_eval<PREC>(P.map[a], g, l, p)) {
             ep[0] += p[0];
             for (int d = 0; d < 3; d++) f[d] += p[1 + d];
         } else {
             bad = 1.0;
         }
     }
-    // sorbate-sorbate LJ against the listed partners in site order: the list
-    // holds every partner within hicut, so the sums are those of the loop over
-    // all sites of the other molecules that skips pairs beyond hicut and
-    // switched-off type pairs
-    double el = 0.0;
-    if (PREC == MH_PREC_FP64) {
-        const double *pp = P.pp64[a * HS];
-        list_loop(nbl, (unsigned)s, n, (unsigned)cap, [&](int j) {
-            const double *pr = pp + 4 * ru[j].w;
-            const double sx = fold64(ri[0] - r[3 * j], P.full[0]);
-            const double sy = fold64(ri[1] - r[3 * j + 1], P.full[1]);
-            const double sz = fold64(ri[2] - r[3 * j + 2], P.full[2]);
-            const double r2 = sx * sx + sy * sy + sz * sz;
-            if (r2 > pr[2]) return;
-            if (r2 < pr[3]) bad = 1.0;
-            const double r2i = 1.0 / r2, r6i = r2i * r2i * r2i, r12i = r6i * r6i;
-            el += pr[0] * r12i - pr[1] * r6i;
-            const double fm = (12.0 * pr[0] * r12i - 6.0 * pr[1] * r6i) * r2i;
-            f[0] += sx * fm;
-            f[1] += sy * fm;
-            f[2] += sz * fm;
-        });
-    } else {
-#pragma clang fp contract(fast)
-        const float ux = P.fxu[0], uy = P.fxu[1], uz = P.fxu[2];
-        const uint4 pi = ru[s];
-        const float4 *pp = P.pp32 + a * HS;
-        float elf = 0.0f, fxf = 0.0f, fyf = 0.0f, fzf = 0.0f;
-        bool badf = false;
-        list_loop(nbl, (unsigned)s, n, (unsigned)cap, [&](int j) {
-            const uint4 pj = ru[j];
-            const float x = (float)(int)(pi.x - pj.x) * ux, y = (float)(int)(pi.y - pj.y) * uy,
-                        z = (float)(int)(pi.z - pj.z) * uz;
-            const float r2 = x * x + y * y + z * z;
-            const float4 pr = pp[pj.w];
-            const bool in = !(r2 > pr.z);
-            badf |= in && r2 < pr.w;
-            // A/r^12 - B/r^6 and its force factor (12 A/r^12 - 6 B/r^6)/r^2
-            const float r2i = in ? rcp_fast(r2) : 0.0f, r6i = r2i * r2i * r2i;
-            const float ta = pr.x * r6i * r6i, tb = pr.y * r6i, de = ta - tb;
-            elf += de;
-            const float fm = (de + ta) * (6.0f * r2i);
-            fxf += x * fm;
-            fyf += y * fm;
-            fzf += z * fm;
-        });
-        if (badf) bad = 1.0;
-        el = elf;
-        f[0] += fxf;
-        f[1] += fyf;
-        f[2] += fzf;
-    }
-    ep[1] += 0.5 * el;  // each pair is seen from both of its sites
-    if (PREC == MH_PREC_FP64) bonded_site(P, rp + 3 * (m * ns), a, fb, eb);
-    for (int k = 0; k < 3; k++) ep[2 + k] += eb[k];
-    for (int d = 0; d < 3; d++) f[d] += fb[d];
+    for (int d = 0; d < 3; d++) f[d] = quad_sum(f[d]);
 }
 
-// energy and forces of the configuration.  With Fo the forces are stored
-// there; otherwise each site's acceleration goes to ga and, after a
-// velocity-Verlet step (step > 0), its velocity gv takes the second half
-// kick.  ke = block total of m v^2 with the velocities after this call.
+// energy and forces of the configuration: each site's acceleration goes to ga
+// and, after a velocity-Verlet step (step > 0), its velocity gv takes the
+// second half kick.  ke = block total of m v^2 with the velocities after this call.
 // Accelerations and velocities written for an evaluation that fails are not
 // used (the move or run ends there).  With MD, parts = block totals of the
 // energy parts and mom = total momentum sum m v; without, parts[0] = the
 // total energy.
+//
+// Two kinds of tasks of one wave each: the bonded terms of 64 sites (a lane
+// per site) and the map and LJ terms of 16 sites (a quad per site); the waves
+// take them in turn, the longer bonded ones first, and fa / fb (LDS where
+// they fit) carry the forces to the lane that moves the site.  One lane per
+// site left one wave on each SIMD for a chain of 6000 FP64 instructions
+// (38 us a step of 240 sites in FP64).
 template <int NT, int PREC, bool MD>
 __device__ void hmc_forces_parts(const HDev &P, const double *rp, const double *r, const uint4 *ru,
-                                 const float4 *nb, int N, const uint16_t *nbl, int cap, double *gv, double *ga,
-                                 double *Fo, int step, double (&parts)[kParts], int &fail, double &ke,
+                                 const float4 *nb, int N, const uint16_t *nbl, int cap, double *fa, double *gv,
+                                 double *ga, int step, double (&parts)[kParts], int &fail, double &ke,
                                  double (&mom)[3], double *red) {
     const int ns = P.ns, nsite = N * ns;
+    double *fb = fa + 3 * cap;
     double ep[kParts] = {0.0, 0.0, 0.0, 0.0, 0.0}, bad = 0.0, k2 = 0.0, px = 0.0, py = 0.0, pz = 0.0;
+    const int lane = threadIdx.x & 63, bonded = (nsite + 63) / 64, tasks = bonded + (nsite * kQuad + 63) / 64;
+#pragma unroll 1
+    for (int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < tasks; t += NT / 64) {
+        if (t < bonded) {
+            const int s = t * 64 + lane;
+            if (s < nsite) {
+                const int m = s / ns;
+                double f[3] = {0.0, 0.0, 0.0}, eb[3] = {0.0, 0.0, 0.0};
+                bonded_site(P, rp + 3 * (m * ns), s - m * ns, f, eb);
+                for (int k = 0; k < 3; k++) {
+                    ep[2 + k] += eb[k];
+                    fb[3 * s + k] = f[k];
+                }
+            }
+        } else {
+            const int w = (t - bonded) * 64 + lane, s = w / kQuad, l = w % kQuad;
+            if (s < nsite) {
+                double f[3];
+                site_force<PREC>(P, r, ru, nbl, cap, s, l, __float_as_int(nb[s].w), f, ep, bad);
+                if (l < 3) fa[3 * s + l] = l == 0 ? f[0] : (l == 1 ? f[1] : f[2]);
+            }
+        }
+    }
+    __syncthreads();
 #pragma unroll 1
     for (int s = threadIdx.x; s < nsite; s += NT) {
-        double f[3];
-        site_force<PREC>(P, rp, r, ru, nbl, cap, s, __float_as_int(nb[s].w), f, ep, bad);
-        if (Fo) {
-            for (int i = 0; i < 3; i++) Fo[3 * s + i] = f[i];
-            continue;
-        }
         const int at = s - (s / ns) * ns;
         double v[3];
         for (int i = 0; i < 3; i++) {
-            const double acc = f[i] * (1.0 / P.mass[at]) * kScaleF;
+            const double acc = (fa[3 * s + i] + fb[3 * s + i]) * (1.0 / P.mass[at]) * kScaleF;
             ga[3 * s + i] = acc;
             v[i] = gv[3 * s + i];
             if (step > 0) {
@@ -560,10 +584,10 @@ __device__ void hmc_forces_parts(const HDev &P, const double *rp, const double *
 // hmc_forces_parts with the total energy U
 template <int NT, int PREC>
 __device__ void hmc_forces(const HDev &P, const double *rp, const double *r, const uint4 *ru, const float4 *nb,
-                           int N, const uint16_t *nbl, int cap, double *gv, double *ga, double *Fo, int step,
+                           int N, const uint16_t *nbl, int cap, double *fa, double *gv, double *ga, int step,
                            double &U, int &fail, double &ke, double *red) {
     double parts[kParts], mom[3];
-    hmc_forces_parts<NT, PREC, false>(P, rp, r, ru, nb, N, nbl, cap, gv, ga, Fo, step, parts, fail, ke, mom, red);
+    hmc_forces_parts<NT, PREC, false>(P, rp, r, ru, nb, N, nbl, cap, fa, gv, ga, step, parts, fail, ke, mom, red);
     U = parts[0];
 }
 
@@ -583,6 +607,7 @@ __global__ void __launch_bounds__(NT) k_hmc(const HDev *__restrict__ Pg, HRep R,
     double *rp = dyn, *r = dyn + (long long)R.cap * 3;
     uint4 *ru = reinterpret_cast<uint4 *>(dyn + (long long)R.cap * 6);
     float4 *nb = reinterpret_cast<float4 *>(ru + R.cap);
+    double *fa = R.fx ? R.fx + 2 * off : reinterpret_cast<double *>(nb + R.cap);
     uint16_t *nbl = R.nbl + (long long)rep * R.cap * R.cap;
     double *gv = R.v + off, *ga = R.a + off;
     for (int i = tid; i < nsite * 3; i += NT) {
@@ -647,7 +672,7 @@ __global__ void __launch_bounds__(NT) k_hmc(const HDev *__restrict__ Pg, HRep R,
             if (__syncthreads_or(moved_far<NT>(rp, nb, nsite))) hmc_lists<NT>(P, ru, rp, N, nbl, R.cap, nb);
             int fl;
             double k2;
-            hmc_forces<NT, PREC>(P, rp, r, ru, nb, N, nbl, R.cap, gv, ga, nullptr, step, U1, fl, k2, red);
+            hmc_forces<NT, PREC>(P, rp, r, ru, nb, N, nbl, R.cap, fa, gv, ga, step, U1, fl, k2, red);
             if (step == 0) {
                 if (ghave && (used & 1u)) gz2 = s_z2;  // written before the block sums
                 if (fl || U1 > P.max_nrg0) {
@@ -739,7 +764,8 @@ __global__ void __launch_bounds__(NT) k_md(const HDev *__restrict__ Pg, HRep R, 
     double *rp = dyn, *r = dyn + (long long)R.cap * 3;
     uint4 *ru = reinterpret_cast<uint4 *>(dyn + (long long)R.cap * 6);
     float4 *nb = reinterpret_cast<float4 *>(ru + R.cap);
-    double *pm = reinterpret_cast<double *>(nb + R.cap);  // [cap][3] site momenta
+    double *fa = R.fx ? R.fx + 2 * off : reinterpret_cast<double *>(nb + R.cap);
+    double *pm = fa;  // [cap][3] site momenta, between two force evaluations
     uint16_t *nbl = R.nbl + (long long)rep * R.cap * R.cap;
     double *gv = R.v + off, *ga = R.a + off;
     for (int i = tid; i < nsite * 3; i += NT) {
@@ -753,7 +779,7 @@ __global__ void __launch_bounds__(NT) k_md(const HDev *__restrict__ Pg, HRep R, 
     double parts[kParts], mom[3], k2;
     int fl, err = 0;
     // accelerations of the start configuration
-    hmc_forces_parts<NT, PREC, true>(P, rp, r, ru, nb, N, nbl, R.cap, gv, ga, nullptr, 0, parts, fl, k2, mom, red);
+    hmc_forces_parts<NT, PREC, true>(P, rp, r, ru, nb, N, nbl, R.cap, fa, gv, ga, 0, parts, fl, k2, mom, red);
     if (fl) err = 2;
     for (int step = 1; step <= nsteps && !err; step++) {
 #pragma unroll 1
@@ -767,8 +793,8 @@ __global__ void __launch_bounds__(NT) k_md(const HDev *__restrict__ Pg, HRep R, 
             put_fx(P, ru, r, s, s - (s / ns) * ns);
         }
         if (__syncthreads_or(moved_far<NT>(rp, nb, nsite))) hmc_lists<NT>(P, ru, rp, N, nbl, R.cap, nb);
-        hmc_forces_parts<NT, PREC, true>(P, rp, r, ru, nb, N, nbl, R.cap, gv, ga, nullptr, step, parts, fl, k2,
-                                         mom, red);
+        hmc_forces_parts<NT, PREC, true>(P, rp, r, ru, nb, N, nbl, R.cap, fa, gv, ga, step, parts, fl, k2, mom,
+                                         red);
         // velverlet_nveIntegrate evaluates with max_nrg = 1000 (velverlet.F90:197-198)
         if (fl || parts[0] + parts[1] + parts[2] + parts[3] + parts[4] > P.max_nrg_md) {
             err = 2;
@@ -808,36 +834,69 @@ __global__ void __launch_bounds__(NT) k_md(const HDev *__restrict__ Pg, HRep R, 
     if (tid == 0 && err) R.err[rep] = err;
 }
 
-// energy and forces of one replica's configuration (tests, checks)
-template <int NT, int PREC>
-__global__ void __launch_bounds__(NT) k_hmc_forces(const HDev *__restrict__ Pg, HRep R, int rep, double *F_out,
-                                                   double *e_out) {
-    extern __shared__ double dyn[];
-    __shared__ HDev P;
-    __shared__ double red[NT / 64 * 4];
-    const int tid = threadIdx.x;
-    for (int i = tid; i < (int)(sizeof(HDev) / 4); i += NT)
-        reinterpret_cast<int *>(&P)[i] = reinterpret_cast<const int *>(Pg)[i];
-    __syncthreads();
+// Energy and forces of one replica's configuration, one workgroup per site:
+// wave 0 the LJ pairs (lanes over all partners) and the map (a quad), wave 1
+// the bonded terms (a lane per term).  out: F [cap][3], then (energy share,
+// failed) [cap][2], then N.  Latency-bound: one workgroup for the whole
+// configuration, lists and all, took 147 us for 320 sites in FP64.
+template <int PREC>
+__global__ void __launch_bounds__(128) k_hmc_forces(const HDev *__restrict__ Pg, HRep R, int rep,
+                                                    double *__restrict__ out) {
+    __shared__ double s_b[4];
+    const HDev &P = *Pg;
+    const int lane = threadIdx.x & 63, s = blockIdx.x;
     const int ns = P.ns, N = R.N[rep], nsite = N * ns;
-    const long long off = (long long)rep * R.cap * 3;
-    double *rp = dyn, *r = dyn + (long long)R.cap * 3;
-    uint4 *ru = reinterpret_cast<uint4 *>(dyn + (long long)R.cap * 6);
-    float4 *nb = reinterpret_cast<float4 *>(ru + R.cap);
-    uint16_t *nbl = R.nbl + (long long)rep * R.cap * R.cap;
-    for (int i = tid; i < nsite * 3; i += NT) {
-        rp[i] = R.rp[off + i];
-        r[i] = R.r[off + i];
+    if (s == 0 && threadIdx.x == 0) out[5 * (long long)R.cap] = N;
+    if (s >= nsite) return;
+    const double *r = R.r + (long long)rep * R.cap * 3, *rp = R.rp + (long long)rep * R.cap * 3;
+    const int m = s / ns, a = s - m * ns;
+    double f[3] = {0.0, 0.0, 0.0}, e = 0.0, bad = 0.0;
+    if (threadIdx.x < 64) {
+        const double rs[3] = {r[3 * s], r[3 * s + 1], r[3 * s + 2]};
+        Corners g;
+        const bool mapped = P.has_map[a] != 0 && lane < kQuad;
+        const bool inside = mapped && hermite_fetch(P.map[a], rs, lane, g);
+        PairSum<PREC> ps(P);
+        const uint4 pi = fx_of(P, rs, a);
+        for (int j = lane; j < nsite; j += 64) {
+            if (j / ns == m) continue;
+            const double rj[3] = {r[3 * j], r[3 * j + 1], r[3 * j + 2]};
+            const int b = j % ns;
+            if (PREC == MH_PREC_FP64) ps.pair64(P, P.pp64[a * HS + b], rs, rj);
+            else ps.pair32(P, P.pp32 + a * HS, pi, fx_of(P, rj, b));
+        }
+        ps.close();
+        if (ps.bad) bad = 1.0;
+        e = 0.5 * ps.el;
+        for (int d = 0; d < 3; d++) f[d] = ps.f[d];
+        if (mapped) {
+            double p[4];
+            if (inside && hermite_eval<PREC>(P.map[a], g, lane, p)) {
+                e += p[0];
+                for (int d = 0; d < 3; d++) f[d] += p[1 + d];
+            } else {
+                bad = 1.0;
+            }
+        }
+    } else {
+        double eb[3] = {0.0, 0.0, 0.0};
+        bonded_site(P, rp + 3 * (m * ns), a, f, eb, lane, 64);
+        e = eb[0] + eb[1] + eb[2];
     }
-    for (int i = tid; i < nsite; i += NT) put_fx(P, ru, R.r + off, i, i % ns);
+    e = wave_sum(e);
+    for (int d = 0; d < 3; d++) f[d] = wave_sum(f[d]);
+    if (threadIdx.x == 64) {
+        for (int d = 0; d < 3; d++) s_b[d] = f[d];
+        s_b[3] = e;
+    }
     __syncthreads();
-    hmc_lists<NT>(P, ru, rp, N, nbl, R.cap, nb);
-    double U, k2;
-    int fl;
-    hmc_forces<NT, PREC>(P, rp, r, ru, nb, N, nbl, R.cap, nullptr, nullptr, F_out, 0, U, fl, k2, red);
-    if (tid == 0) {
-        e_out[0] = U;
-        e_out[1] = fl ? 0.0 : 1.0;
+    if (threadIdx.x < 64) {
+        bad = wave_sum(bad);
+        if (lane == 0) {
+            for (int d = 0; d < 3; d++) out[3 * s + d] = f[d] + s_b[d];
+            out[3 * (long long)R.cap + 2 * s] = e + s_b[3];
+            out[3 * (long long)R.cap + 2 * s + 1] = bad;
+        }
     }
 }
 
@@ -851,6 +910,9 @@ struct mh_hmc {
     size_t lds = 0;
     HDev host;
     DBuf dP;
+    bool fx_lds = true;  // partial forces in LDS (else in fx)
+    DBuf fx, fout;       // fout: output of mh_hmc_energy_forces
+    std::mutex fout_mu;
     DBuf N, err, ix, iy, first, iseed, ghave, gz2, energy, dH, att, acc, fail, rp, r, rp0, r0, v, a, nbl;
     HRep rep() {
         HRep h;
@@ -875,6 +937,7 @@ struct mh_hmc {
         h.a = a.as<double>();
         h.nbl = nbl.as<uint16_t>();
         h.cap = maxN * ns;
+        h.fx = fx_lds ? nullptr : fx.as<double>();
         return h;
     }
 };
@@ -915,12 +978,19 @@ static int launch_hmc(mh_hmc *h, int nmoves) {
 // LDS per site: rp and r (FP64), fixed-point position, list bookkeeping
 constexpr size_t kLdsPerSite = 6 * sizeof(double) + sizeof(uint4) + sizeof(float4);
 
+// partial forces per site (two of them), in LDS where they fit as well
+constexpr size_t kLdsForces = 6 * sizeof(double);
+
 static int plan_hmc(mh_hmc *h) {
     int dev_max = 65536;
     (void)hipDeviceGetAttribute(&dev_max, hipDeviceAttributeMaxSharedMemoryPerBlock, h->ctx->device);
-    h->lds = (size_t)h->maxN * h->ns * kLdsPerSite;
+    const size_t sites = (size_t)h->maxN * h->ns;
+    h->lds = sites * kLdsPerSite;
     MH_CHECK((long long)h->lds + (long long)sizeof(HDev) + 8192 <= dev_max, MH_ECAPACITY,
              "mh_hmc: maxN * nsites too large for LDS (positions of a replica are held in LDS)");
+    h->fx_lds = (long long)(sites * (kLdsPerSite + kLdsForces)) + (long long)sizeof(HDev) + 8192 <= dev_max;
+    if (h->fx_lds) h->lds += sites * kLdsForces;
+    else if (!h->fx.p) return h->fx.alloc(kLdsForces * sites * h->nrep);
     return MH_OK;
 }
 
@@ -1193,7 +1263,8 @@ int mh_hmc_md(mh_hmc *h, int nsteps, double *trace) {
     MH_CHECK(h && nsteps >= 0 && (nsteps == 0 || trace), MH_EINVAL, "mh_hmc_md: bad arguments");
     if (!nsteps) return MH_OK;
     MH_HIP(hipSetDevice(h->ctx->device));
-    const size_t lds = h->lds + (size_t)h->maxN * h->ns * 3 * sizeof(double);
+    // site momenta take the place of the partial forces between evaluations
+    const size_t lds = (size_t)h->maxN * h->ns * (kLdsPerSite + 3 * sizeof(double));
     int dev_max = 65536;
     (void)hipDeviceGetAttribute(&dev_max, hipDeviceAttributeMaxSharedMemoryPerBlock, h->ctx->device);
     MH_CHECK((long long)lds + (long long)sizeof(HDev) + 8192 <= dev_max, MH_ECAPACITY,
@@ -1204,8 +1275,8 @@ int mh_hmc_md(mh_hmc *h, int nsteps, double *trace) {
     if ((rc = dtrace.alloc(8 * nt))) return rc;
     MH_HIP(hipMemsetAsync(dtrace.p, 0, 8 * nt, h->ctx->stream));
     KTimer t(h->ctx, h->prec == MH_PREC_FP32 ? "md32" : "md64");
-    if (h->prec == MH_PREC_FP32) launch_md<MH_PREC_FP32>(h, nsteps, dtrace.as<double>(), lds);
-    else launch_md<MH_PREC_FP64>(h, nsteps, dtrace.as<double>(), lds);
+    if (h->prec == MH_PREC_FP32) launch_md<MH_PREC_FP32>(h, nsteps, dtrace.as<double>(), h->lds);
+    else launch_md<MH_PREC_FP64>(h, nsteps, dtrace.as<double>(), h->lds);
     MH_HIP(hipGetLastError());
     MH_HIP(hipStreamSynchronize(h->ctx->stream));
     t.stop();
@@ -1220,29 +1291,34 @@ int mh_hmc_md(mh_hmc *h, int nsteps, double *trace) {
 int mh_hmc_energy_forces(mh_hmc *h, int rep, double *e, double *F, int *ok) {
     MH_CHECK(h && rep >= 0 && rep < h->nrep && e && ok, MH_EINVAL, "mh_hmc_energy_forces: bad arguments");
     MH_HIP(hipSetDevice(h->ctx->device));
-    DBuf dF, de;
-    int rc;
-    const size_t nc = (size_t)h->maxN * h->ns * 3;
-    if ((rc = dF.alloc(8 * (nc + 1))) || (rc = de.alloc(16))) return rc;
-    HRep R = h->rep();
-    const HDev *P = h->dP.as<HDev>();
-    auto go = [&](auto kern) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)h->lds);
-        hipLaunchKernelGGL(kern, dim3(1), dim3(256), h->lds, h->ctx->stream, P, R, rep, dF.as<double>(),
-                           de.as<double>());
-    };
-    if (h->prec == MH_PREC_FP32) go(k_hmc_forces<256, MH_PREC_FP32>);
-    else go(k_hmc_forces<256, MH_PREC_FP64>);
-    MH_HIP(hipGetLastError());
-    MH_HIP(hipStreamSynchronize(h->ctx->stream));
-    double hv[2];
-    MH_HIP(hipMemcpy(hv, de.p, 16, hipMemcpyDeviceToHost));
-    *e = hv[0];
-    *ok = hv[1] != 0.0;
-    int hn = 0;
-    MH_HIP(hipMemcpy(&hn, h->N.as<int>() + rep, 4, hipMemcpyDeviceToHost));
-    if (F && hn) MH_HIP(hipMemcpy(F, dF.p, 8 * (size_t)hn * h->ns * 3, hipMemcpyDeviceToHost));
+    const size_t cap = (size_t)h->maxN * h->ns, no = 5 * cap + 1;
+    std::vector<double> o(no);
+    {
+        std::lock_guard<std::mutex> lk(h->fout_mu);
+        if (!h->fout.p)
+            if (int rc = h->fout.alloc(8 * no)) return rc;
+        HRep R = h->rep();
+        const HDev *P = h->dP.as<HDev>();
+        hipStream_t st = h->ctx->stream;
+        if (h->prec == MH_PREC_FP32)
+            hipLaunchKernelGGL(k_hmc_forces<MH_PREC_FP32>, dim3((unsigned)cap), dim3(128), 0, st, P, R, rep,
+                               h->fout.as<double>());
+        else
+            hipLaunchKernelGGL(k_hmc_forces<MH_PREC_FP64>, dim3((unsigned)cap), dim3(128), 0, st, P, R, rep,
+                               h->fout.as<double>());
+        MH_HIP(hipGetLastError());
+        MH_HIP(hipMemcpyAsync(o.data(), h->fout.p, 8 * no, hipMemcpyDeviceToHost, st));
+        MH_HIP(hipStreamSynchronize(st));
+    }
+    const size_t nsite = (size_t)o[5 * cap] * h->ns;
+    double U = 0.0, bad = 0.0;
+    for (size_t s = 0; s < nsite; s++) {
+        U += o[3 * cap + 2 * s];
+        bad += o[3 * cap + 2 * s + 1];
+    }
+    *e = U;
+    *ok = bad == 0.0;
+    if (F) std::memcpy(F, o.data(), 8 * 3 * nsite);
     return MH_OK;
 }
 
