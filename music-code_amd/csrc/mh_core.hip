@@ -2,6 +2,7 @@
 #include <cmath>
 #include <cstring>
 #include <cstdio>
+#include <mutex>
 
 #include "mh_internal.h"
 
@@ -10,10 +11,150 @@ namespace mh {
 static thread_local std::string g_err;
 void set_error(const std::string &msg) { g_err = msg; }
 
+namespace {
+struct Pool {
+    struct Block {
+        void *p;
+        size_t n;
+    };
+    std::vector<Block> blocks;  // oldest first
+    size_t bytes = 0;
+    int contexts = 0;
+};
+std::mutex g_pool_mu;
+std::map<int, Pool> g_pools;
+std::vector<Pool::Block> g_pins;  // idle pinned blocks
+int g_contexts = 0;
+
+void pool_flush(Pool &q) {
+    for (auto &b : q.blocks) (void)hipFree(b.p);
+    q.blocks.clear();
+    q.bytes = 0;
+}
+}  // namespace
+
+int pool_take(DBuf &b, size_t bytes) {
+    b.release();
+    int dev = 0;
+    MH_HIP(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lk(g_pool_mu);
+        Pool &q = g_pools[dev];
+        size_t best = q.blocks.size();
+        for (size_t i = 0; i < q.blocks.size(); i++) {
+            const size_t n = q.blocks[i].n;
+            if (n < bytes || n > 2 * bytes + (1 << 20)) continue;
+            if (best == q.blocks.size() || n < q.blocks[best].n) best = i;
+        }
+        if (best < q.blocks.size()) {
+            b.p = q.blocks[best].p;
+            b.n = q.blocks[best].n;
+            q.bytes -= b.n;
+            q.blocks.erase(q.blocks.begin() + best);
+            return MH_OK;
+        }
+    }
+    return b.alloc(bytes);
+}
+
+void pool_give(DBuf &b) {
+    if (!b.p) return;
+    int dev = 0;
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    if (hipGetDevice(&dev) == hipSuccess && g_pools[dev].contexts > 0 && b.n <= kPoolBytes / 2) {
+        Pool &q = g_pools[dev];
+        q.blocks.push_back({b.p, b.n});
+        q.bytes += b.n;
+        b.p = nullptr;
+        b.n = 0;
+        while (q.bytes > kPoolBytes || q.blocks.size() > kPoolBlocks) {
+            (void)hipFree(q.blocks.front().p);
+            q.bytes -= q.blocks.front().n;
+            q.blocks.erase(q.blocks.begin());
+        }
+        return;
+    }
+    b.release();
+}
+
+static int pin_take(size_t bytes, Pool::Block &b) {
+    {
+        std::lock_guard<std::mutex> lk(g_pool_mu);
+        for (size_t i = 0; i < g_pins.size(); i++)
+            if (g_pins[i].n >= bytes) {
+                b = g_pins[i];
+                g_pins.erase(g_pins.begin() + i);
+                return MH_OK;
+            }
+    }
+    b.n = bytes > kPinLeast ? bytes : kPinLeast;
+    MH_HIP(hipHostMalloc(&b.p, b.n, hipHostMallocPortable));
+    return MH_OK;
+}
+
+static void pin_give(const Pool::Block &b) {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    if (b.n <= kPinBytes && g_pins.size() < kPinBlocks && g_contexts > 0) g_pins.push_back(b);
+    else (void)hipHostFree(b.p);
+}
+
+void pool_ctx(int device, int change) {
+    bool first = false;
+    {
+        std::lock_guard<std::mutex> lk(g_pool_mu);
+        Pool &q = g_pools[device];
+        q.contexts += change;
+        g_contexts += change;
+        if (q.contexts == 0) pool_flush(q);
+        if (g_contexts == 0) {
+            for (auto &b : g_pins) (void)hipHostFree(b.p);
+            g_pins.clear();
+        }
+        first = change > 0 && g_pins.empty();
+    }
+    Pool::Block b;
+    if (first && pin_take(kPinLeast, b) == MH_OK) pin_give(b);
+}
+
+int readback(hipStream_t st, const std::vector<Copy> &items) {
+    auto up = [](size_t n) { return (n + 63) / 64 * 64; };
+    size_t total = 0, o = 0;
+    for (auto &i : items) total += up(i.n);
+    Pool::Block pin;
+    if (int rc = pin_take(total, pin)) return rc;
+    hipError_t e = hipSuccess;
+    for (auto &i : items) {
+        if (i.n && e == hipSuccess) e = hipMemcpyAsync((char *)pin.p + o, i.src, i.n, hipMemcpyDeviceToHost, st);
+        o += up(i.n);
+    }
+    const hipError_t w = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = w;
+    o = 0;
+    for (auto &i : items) {
+        if (i.n && e == hipSuccess) std::memcpy(i.dst, (char *)pin.p + o, i.n);
+        o += up(i.n);
+    }
+    pin_give(pin);
+    if (e != hipSuccess) {
+        set_error(std::string("copy to the host: ") + hipGetErrorString(e));
+        return MH_EHIP;
+    }
+    return MH_OK;
+}
+
 int DBuf::alloc(size_t bytes) {
     release();
     if (bytes == 0) bytes = 16;
     hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) {  // give the kept blocks back and try again
+        (void)hipGetLastError();
+        {
+            int dev = 0;
+            std::lock_guard<std::mutex> lk(g_pool_mu);
+            if (hipGetDevice(&dev) == hipSuccess) pool_flush(g_pools[dev]);
+        }
+        e = hipMalloc(&p, bytes);
+    }
     if (e != hipSuccess) {
         p = nullptr;
         set_error(std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
@@ -141,6 +282,7 @@ int mh_ctx_create(int device, mh_ctx **out) {
         set_error(std::string("hipStreamCreate: ") + hipGetErrorString(e));
         return MH_EHIP;
     }
+    pool_ctx(device, 1);
     *out = c;
     return MH_OK;
 }
@@ -153,6 +295,7 @@ int mh_ctx_destroy(mh_ctx *ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         ctx->ws.clear();
         (void)hipStreamDestroy(ctx->stream);
+        pool_ctx(ctx->device, -1);
         delete ctx;
     }
     return MH_OK;
@@ -193,12 +336,15 @@ int mh_framework_upload(mh_ctx *ctx, int natoms, const double *xyz, const int *t
     ctx->ew.set = false;
     if (natoms == 0) return MH_OK;  // a cell without framework atoms (sorbate-only systems)
     int rc;
-    if ((rc = ctx->xyz.alloc(sizeof(double) * 3 * natoms))) return rc;
-    if ((rc = ctx->type.alloc(sizeof(int) * natoms))) return rc;
-    if ((rc = ctx->q.alloc(sizeof(double) * natoms))) return rc;
-    MH_HIP(hipMemcpy(ctx->xyz.p, ctx->hxyz.data(), sizeof(double) * 3 * natoms, hipMemcpyHostToDevice));
-    MH_HIP(hipMemcpy(ctx->type.p, type, sizeof(int) * natoms, hipMemcpyHostToDevice));
-    MH_HIP(hipMemcpy(ctx->q.p, ctx->hq.data(), sizeof(double) * natoms, hipMemcpyHostToDevice));
+    // arrays that are large enough are written again, on the context's stream
+    const size_t nd = sizeof(double) * natoms, ni = sizeof(int) * natoms;
+    if (ctx->xyz.n < 3 * nd && (rc = ctx->xyz.alloc(3 * nd))) return rc;
+    if (ctx->type.n < ni && (rc = ctx->type.alloc(ni))) return rc;
+    if (ctx->q.n < nd && (rc = ctx->q.alloc(nd))) return rc;
+    MH_HIP(hipMemcpyAsync(ctx->xyz.p, ctx->hxyz.data(), 3 * nd, hipMemcpyHostToDevice, ctx->stream));
+    MH_HIP(hipMemcpyAsync(ctx->type.p, ctx->htype.data(), ni, hipMemcpyHostToDevice, ctx->stream));
+    MH_HIP(hipMemcpyAsync(ctx->q.p, ctx->hq.data(), nd, hipMemcpyHostToDevice, ctx->stream));
+    MH_HIP(hipStreamSynchronize(ctx->stream));
     return MH_OK;
 }
 
@@ -389,24 +535,23 @@ int mh_ewald_set(mh_ctx *ctx, double kappa_param, int kmax, double locut, int si
     double iVolPi = ialpha * ibeta * igamma / kPi;
     const int side = 2 * kmax + 1;
     const int ncand = side * side * side;
-    DBuf keep, cs, csi, ck;
+    // candidates: s, si, k, keep in one block, one copy back
+    PoolBuf cand;
     int rc;
-    if ((rc = keep.alloc(ncand))) return rc;
-    if ((rc = cs.alloc(sizeof(double) * ncand))) return rc;
-    if ((rc = csi.alloc(sizeof(double) * ncand))) return rc;
-    if ((rc = ck.alloc(sizeof(double) * 3 * ncand))) return rc;
+    const size_t cb = sizeof(double) * 5 * (size_t)ncand + ncand;
+    if ((rc = cand.take(cb))) return rc;
+    double *cs = cand.as<double>(), *csi = cs + ncand, *ck = csi + ncand;
+    uint8_t *keep = reinterpret_cast<uint8_t *>(ck + 3 * (size_t)ncand);
     hipLaunchKernelGGL(k_sfactor, dim3((ncand / 2 + 4) / 4), dim3(256), 0, ctx->stream, kmax,
                        ctx->natoms, ctx->xyz.as<double>(), ctx->q.as<double>(), ialpha, ibeta,
-                       igamma, ikapPiSq, iVolPi, locut, keep.as<uint8_t>(), cs.as<double>(),
-                       csi.as<double>(), ck.as<double>());
+                       igamma, ikapPiSq, iVolPi, locut, keep, cs, csi, ck);
     MH_HIP(hipGetLastError());
-    std::vector<uint8_t> hkeep(ncand);
-    std::vector<double> hs(ncand), hsi(ncand), hk(3 * (size_t)ncand);
-    MH_HIP(hipMemcpyAsync(hkeep.data(), keep.p, ncand, hipMemcpyDeviceToHost, ctx->stream));
-    MH_HIP(hipMemcpyAsync(hs.data(), cs.p, sizeof(double) * ncand, hipMemcpyDeviceToHost, ctx->stream));
-    MH_HIP(hipMemcpyAsync(hsi.data(), csi.p, sizeof(double) * ncand, hipMemcpyDeviceToHost, ctx->stream));
-    MH_HIP(hipMemcpyAsync(hk.data(), ck.p, sizeof(double) * 3 * ncand, hipMemcpyDeviceToHost, ctx->stream));
+    std::vector<double> hc(5 * (size_t)ncand + (ncand + 7) / 8);
+    MH_HIP(hipMemcpyAsync(hc.data(), cs, cb, hipMemcpyDeviceToHost, ctx->stream));
     MH_HIP(hipStreamSynchronize(ctx->stream));
+    cand.idle = true;
+    const double *hs = hc.data(), *hsi = hs + ncand, *hk = hsi + ncand;
+    const uint8_t *hkeep = reinterpret_cast<const uint8_t *>(hk + 3 * (size_t)ncand);
     // ordered compaction of the accepted vectors (reference order x,y,z)
     ew.hk.clear();
     ew.hs.clear();
@@ -425,16 +570,10 @@ int mh_ewald_set(mh_ctx *ctx, double kappa_param, int kmax, double locut, int si
     ew.nk = (int)ew.hs.size();
     MH_CHECK(ew.nk <= 50000, MH_ECAPACITY,
              "mh_ewald_set: more than nkmax = 50000 k vectors (ewald.F90:134)");
-    if ((rc = ew.k.alloc(sizeof(double) * 3 * (ew.nk + 1)))) return rc;
-    if ((rc = ew.s.alloc(sizeof(double) * (ew.nk + 1)))) return rc;
-    if ((rc = ew.si.alloc(sizeof(double) * (ew.nk + 1)))) return rc;
-    if ((rc = ew.ccoef.alloc(sizeof(double) * 2 * ncand))) return rc;
-    if (ew.nk) {
-        MH_HIP(hipMemcpy(ew.k.p, ew.hk.data(), sizeof(double) * 3 * ew.nk, hipMemcpyHostToDevice));
-        MH_HIP(hipMemcpy(ew.s.p, ew.hs.data(), sizeof(double) * ew.nk, hipMemcpyHostToDevice));
-        MH_HIP(hipMemcpy(ew.si.p, ew.hsi.data(), sizeof(double) * ew.nk, hipMemcpyHostToDevice));
-    }
-    MH_HIP(hipMemcpy(ew.ccoef.p, grid.data(), sizeof(double) * 2 * ncand, hipMemcpyHostToDevice));
+    const size_t gb = sizeof(double) * 2 * (size_t)ncand;
+    if (ew.ccoef.n < gb && (rc = ew.ccoef.alloc(gb))) return rc;
+    MH_HIP(hipMemcpyAsync(ew.ccoef.p, grid.data(), gb, hipMemcpyHostToDevice, ctx->stream));
+    MH_HIP(hipStreamSynchronize(ctx->stream));
     ew.set = true;
     if (nk_out) *nk_out = ew.nk;
     return MH_OK;

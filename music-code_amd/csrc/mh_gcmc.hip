@@ -2616,10 +2616,10 @@ int mh_gcmc_run(mh_gcmc *g, int nsteps) {
     KTimer t(g->ctx, g->prec == MH_PREC_FP32 ? "gcmc32" : "gcmc64");
     launch_any(g, nsteps);
     MH_HIP(hipGetLastError());
-    MH_HIP(hipStreamSynchronize(g->ctx->stream));
-    t.stop();
     std::vector<int> err(g->nrep);
-    MH_HIP(hipMemcpy(err.data(), g->err.p, 4 * g->nrep, hipMemcpyDeviceToHost));
+    const int rrc = readback(g->ctx->stream, {{err.data(), g->err.p, 4 * (size_t)g->nrep}});
+    t.stop();
+    if (rrc) return rrc;
     for (int i = 0; i < g->nrep; i++) {
         MH_CHECK(err[i] != 2, MH_ECAPACITY, "mh_gcmc_run: a replica reached maxN molecules");
         MH_CHECK(err[i] != 4, MH_ESTATE,
@@ -2696,15 +2696,31 @@ int mh_gcmc_get_state(mh_gcmc *g, int32_t *N, double *energy, double *sumN, int6
     MH_CHECK(g, MH_EINVAL, "mh_gcmc_get_state: g is NULL");
     MH_HIP(hipSetDevice(g->ctx->device));
     const size_t R = g->nrep;
-    int rc;
-    if (N && (rc = spc_gather(g, g->N, 4, N))) return rc;
-    if (energy) MH_HIP(hipMemcpy(energy, g->energy.p, 8 * R, hipMemcpyDeviceToHost));
-    if (sumN && (rc = spc_gather(g, g->sumN, 8, sumN))) return rc;
-    if (nsteps) MH_HIP(hipMemcpy(nsteps, g->nsteps.p, 8 * R, hipMemcpyDeviceToHost));
-    if (att && (rc = spc_gather(g, g->att, 32, att))) return rc;
-    if (acc && (rc = spc_gather(g, g->acc, 32, acc))) return rc;
-    if (rng_ix) MH_HIP(hipMemcpy(rng_ix, g->ix.p, 4 * R, hipMemcpyDeviceToHost));
-    if (rng_iy) MH_HIP(hipMemcpy(rng_iy, g->iy.p, 4 * R, hipMemcpyDeviceToHost));
+    // per-species arrays come whole, the addressed species is picked out
+    std::vector<Copy> it;
+    std::vector<std::vector<char>> whole(4);
+    auto spc = [&](void *dst, const DBuf &b, size_t elem, int k) {
+        if (!dst) return;
+        whole[k].resize(elem * GSPC * R);
+        it.push_back({whole[k].data(), b.p, whole[k].size()});
+    };
+    auto get = [&](void *dst, const DBuf &b, size_t elem) {
+        if (dst) it.push_back({dst, b.p, elem * R});
+    };
+    spc(N, g->N, 4, 0);
+    spc(sumN, g->sumN, 8, 1);
+    spc(att, g->att, 32, 2);
+    spc(acc, g->acc, 32, 3);
+    get(energy, g->energy, 8);
+    get(nsteps, g->nsteps, 8);
+    get(rng_ix, g->ix, 4);
+    get(rng_iy, g->iy, 4);
+    if (int rc = readback(g->ctx->stream, it)) return rc;
+    void *dst[4] = {N, sumN, att, acc};
+    const size_t el[4] = {4, 8, 32, 32};
+    for (int k = 0; k < 4; k++)
+        for (size_t r = 0; dst[k] && r < R; r++)
+            std::memcpy((char *)dst[k] + r * el[k], whole[k].data() + (r * GSPC + g->sel) * el[k], el[k]);
     return MH_OK;
 }
 

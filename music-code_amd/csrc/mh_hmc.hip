@@ -913,6 +913,7 @@ struct mh_hmc {
     bool fx_lds = true;  // partial forces in LDS (else in fx)
     DBuf fx, fout;       // fout: output of mh_hmc_energy_forces
     std::mutex fout_mu;
+    std::vector<int> hN;  // molecules per replica (moves and dynamics keep them)
     DBuf N, err, ix, iy, first, iseed, ghave, gz2, energy, dH, att, acc, fail, rp, r, rp0, r0, v, a, nbl;
     HRep rep() {
         HRep h;
@@ -1032,6 +1033,7 @@ int mh_hmc_create(mh_ctx *ctx, const mh_hmc_params *p, int nrep, const int32_t *
     std::unique_ptr<mh_hmc> h(new mh_hmc());
     h->ctx = ctx;
     h->nrep = nrep;
+    h->hN.assign(nrep, 0);
     h->maxN = maxN;
     h->ns = p->nsites;
     h->prec = p->precision;
@@ -1183,6 +1185,7 @@ int mh_hmc_set_config(mh_hmc *h, int rep, int n, const double *rp) {
         MH_HIP(hipMemcpy(h->r.as<double>() + off, r.data(), 8 * nc, hipMemcpyHostToDevice));
     }
     MH_HIP(hipMemcpy(h->N.as<int>() + rep, &n, 4, hipMemcpyHostToDevice));
+    h->hN[rep] = n;
     double e = 0.0;
     int ok = 1;
     int rc = mh_hmc_energy_forces(h, rep, &e, nullptr, &ok);
@@ -1199,10 +1202,10 @@ int mh_hmc_run(mh_hmc *h, int nmoves) {
     int rc = h->prec == MH_PREC_FP32 ? launch_hmc<MH_PREC_FP32>(h, nmoves) : launch_hmc<MH_PREC_FP64>(h, nmoves);
     if (rc) return rc;
     MH_HIP(hipGetLastError());
-    MH_HIP(hipStreamSynchronize(h->ctx->stream));
-    t.stop();
     std::vector<int> err(h->nrep);
-    MH_HIP(hipMemcpy(err.data(), h->err.p, 4 * h->nrep, hipMemcpyDeviceToHost));
+    rc = readback(h->ctx->stream, {{err.data(), h->err.p, 4 * (size_t)h->nrep}});
+    t.stop();
+    if (rc) return rc;
     for (int i = 0; i < h->nrep; i++)
         MH_CHECK(err[i] == 0, MH_ESTATE, "mh_hmc_run: a replica's start configuration failed to evaluate");
     return MH_OK;
@@ -1213,35 +1216,39 @@ int mh_hmc_get_state(mh_hmc *h, int32_t *N, double *energy, int64_t *att, int64_
     MH_CHECK(h, MH_EINVAL, "mh_hmc_get_state: h is NULL");
     MH_HIP(hipSetDevice(h->ctx->device));
     const size_t R = h->nrep;
-    if (N) MH_HIP(hipMemcpy(N, h->N.p, 4 * R, hipMemcpyDeviceToHost));
-    if (energy) MH_HIP(hipMemcpy(energy, h->energy.p, 8 * R, hipMemcpyDeviceToHost));
-    if (att) MH_HIP(hipMemcpy(att, h->att.p, 8 * R, hipMemcpyDeviceToHost));
-    if (acc) MH_HIP(hipMemcpy(acc, h->acc.p, 8 * R, hipMemcpyDeviceToHost));
-    if (fail) MH_HIP(hipMemcpy(fail, h->fail.p, 8 * R, hipMemcpyDeviceToHost));
-    if (last_dH) MH_HIP(hipMemcpy(last_dH, h->dH.p, 8 * R, hipMemcpyDeviceToHost));
-    if (rng_ix) MH_HIP(hipMemcpy(rng_ix, h->ix.p, 4 * R, hipMemcpyDeviceToHost));
-    if (rng_iy) MH_HIP(hipMemcpy(rng_iy, h->iy.p, 4 * R, hipMemcpyDeviceToHost));
+    std::vector<Copy> it;
+    auto get = [&](void *dst, const DBuf &b, size_t elem) {
+        if (dst) it.push_back({dst, b.p, elem * R});
+    };
+    get(N, h->N, 4);
+    get(energy, h->energy, 8);
+    get(att, h->att, 8);
+    get(acc, h->acc, 8);
+    get(fail, h->fail, 8);
+    get(last_dH, h->dH, 8);
+    get(rng_ix, h->ix, 4);
+    get(rng_iy, h->iy, 4);
+    if (int rc = readback(h->ctx->stream, it)) return rc;
     return MH_OK;
 }
 
 int mh_hmc_get_config(mh_hmc *h, int rep, int *n, double *rp, double *r) {
     MH_CHECK(h && rep >= 0 && rep < h->nrep && n, MH_EINVAL, "mh_hmc_get_config: bad arguments");
     MH_HIP(hipSetDevice(h->ctx->device));
-    int hn = 0;
-    MH_HIP(hipMemcpy(&hn, h->N.as<int>() + rep, 4, hipMemcpyDeviceToHost));
+    const int hn = h->hN[rep];
     *n = hn;
     const size_t nc = (size_t)hn * h->ns * 3, off = (size_t)rep * h->maxN * h->ns * 3;
-    if (nc && rp) MH_HIP(hipMemcpy(rp, h->rp.as<double>() + off, 8 * nc, hipMemcpyDeviceToHost));
-    if (nc && r) MH_HIP(hipMemcpy(r, h->r.as<double>() + off, 8 * nc, hipMemcpyDeviceToHost));
-    return MH_OK;
+    std::vector<Copy> it;
+    if (nc && rp) it.push_back({rp, h->rp.as<double>() + off, 8 * nc});
+    if (nc && r) it.push_back({r, h->r.as<double>() + off, 8 * nc});
+    return readback(h->ctx->stream, it);
 }
 
 int mh_hmc_set_velocities(mh_hmc *h, int rep, int n, const double *v) {
     MH_CHECK(h && rep >= 0 && rep < h->nrep && n >= 0 && (n == 0 || v), MH_EINVAL,
              "mh_hmc_set_velocities: bad arguments");
     MH_HIP(hipSetDevice(h->ctx->device));
-    int hn = 0;
-    MH_HIP(hipMemcpy(&hn, h->N.as<int>() + rep, 4, hipMemcpyDeviceToHost));
+    const int hn = h->hN[rep];
     MH_CHECK(n == hn, MH_EINVAL, "mh_hmc_set_velocities: n differs from the replica's molecule count");
     const size_t nc = (size_t)n * h->ns * 3, off = (size_t)rep * h->maxN * h->ns * 3;
     if (nc) MH_HIP(hipMemcpy(h->v.as<double>() + off, v, 8 * nc, hipMemcpyHostToDevice));
@@ -1251,12 +1258,12 @@ int mh_hmc_set_velocities(mh_hmc *h, int rep, int n, const double *v) {
 int mh_hmc_get_velocities(mh_hmc *h, int rep, int *n, double *v) {
     MH_CHECK(h && rep >= 0 && rep < h->nrep && n, MH_EINVAL, "mh_hmc_get_velocities: bad arguments");
     MH_HIP(hipSetDevice(h->ctx->device));
-    int hn = 0;
-    MH_HIP(hipMemcpy(&hn, h->N.as<int>() + rep, 4, hipMemcpyDeviceToHost));
+    const int hn = h->hN[rep];
     *n = hn;
     const size_t nc = (size_t)hn * h->ns * 3, off = (size_t)rep * h->maxN * h->ns * 3;
-    if (nc && v) MH_HIP(hipMemcpy(v, h->v.as<double>() + off, 8 * nc, hipMemcpyDeviceToHost));
-    return MH_OK;
+    std::vector<Copy> it;
+    if (nc && v) it.push_back({v, h->v.as<double>() + off, 8 * nc});
+    return readback(h->ctx->stream, it);
 }
 
 int mh_hmc_md(mh_hmc *h, int nsteps, double *trace) {
@@ -1270,19 +1277,19 @@ int mh_hmc_md(mh_hmc *h, int nsteps, double *trace) {
     MH_CHECK((long long)lds + (long long)sizeof(HDev) + 8192 <= dev_max, MH_ECAPACITY,
              "mh_hmc_md: maxN * nsites too large for LDS");
     const size_t nt = (size_t)h->nrep * nsteps * MH_MD_NQ;
-    DBuf dtrace;
+    PoolBuf dtrace;
     int rc;
-    if ((rc = dtrace.alloc(8 * nt))) return rc;
+    if ((rc = dtrace.take(8 * nt))) return rc;
     MH_HIP(hipMemsetAsync(dtrace.p, 0, 8 * nt, h->ctx->stream));
     KTimer t(h->ctx, h->prec == MH_PREC_FP32 ? "md32" : "md64");
     if (h->prec == MH_PREC_FP32) launch_md<MH_PREC_FP32>(h, nsteps, dtrace.as<double>(), h->lds);
     else launch_md<MH_PREC_FP64>(h, nsteps, dtrace.as<double>(), h->lds);
     MH_HIP(hipGetLastError());
-    MH_HIP(hipStreamSynchronize(h->ctx->stream));
-    t.stop();
-    MH_HIP(hipMemcpy(trace, dtrace.p, 8 * nt, hipMemcpyDeviceToHost));
     std::vector<int> err(h->nrep);
-    MH_HIP(hipMemcpy(err.data(), h->err.p, 4 * h->nrep, hipMemcpyDeviceToHost));
+    rc = readback(h->ctx->stream, {{trace, dtrace.p, 8 * nt}, {err.data(), h->err.p, 4 * (size_t)h->nrep}});
+    t.stop();
+    if (rc) return rc;
+    dtrace.idle = true;
     for (int i = 0; i < h->nrep; i++)
         MH_CHECK(err[i] == 0, MH_ESTATE, "mh_hmc_md: a replica's energy evaluation failed (overlap or off-map site)");
     return MH_OK;
@@ -1307,8 +1314,7 @@ int mh_hmc_energy_forces(mh_hmc *h, int rep, double *e, double *F, int *ok) {
             hipLaunchKernelGGL(k_hmc_forces<MH_PREC_FP64>, dim3((unsigned)cap), dim3(128), 0, st, P, R, rep,
                                h->fout.as<double>());
         MH_HIP(hipGetLastError());
-        MH_HIP(hipMemcpyAsync(o.data(), h->fout.p, 8 * no, hipMemcpyDeviceToHost, st));
-        MH_HIP(hipStreamSynchronize(st));
+        if (int rc = readback(st, {{o.data(), h->fout.p, 8 * no}})) return rc;
     }
     const size_t nsite = (size_t)o[5 * cap] * h->ns;
     double U = 0.0, bad = 0.0;

@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -41,6 +42,39 @@ struct DBuf {
     template <class T> T *as() const { return reinterpret_cast<T *>(p); }
 };
 
+// Device blocks kept for the next call of the same kind (hipMalloc and hipFree
+// of a map's arrays cost more than a small map's kernels).  One list per
+// device for every context and thread, at most kPoolBytes in kPoolBlocks
+// blocks, freed with the device's last context and when an allocation fails.
+// pool_give: the block must be idle (the work that used it waited for).
+constexpr size_t kPoolBytes = (size_t)4 << 30, kPoolBlocks = 16;
+int pool_take(DBuf &b, size_t bytes);
+void pool_give(DBuf &b);
+void pool_ctx(int device, int change);  // contexts of a device: +1 / -1
+// a block of the pool for the length of a call; idle: its stream was waited
+// for (an early return waits for the device, as hipFree does)
+struct PoolBuf : DBuf {
+    bool idle = false;
+    int take(size_t bytes) { return pool_take(*this, bytes); }
+    ~PoolBuf() {
+        if (p && !idle) (void)hipDeviceSynchronize();
+        pool_give(*this);
+    }
+};
+
+// Device arrays read back together: asynchronous copies into pinned memory,
+// one wait, then the caller's arrays (a synchronous copy each costs a wait).
+// The pinned blocks are the process's (allocating one costs 400 us): each call
+// takes one for itself, at most kPinBlocks of up to kPinBytes are kept, until
+// the last context is gone.
+constexpr size_t kPinBlocks = 8, kPinBytes = (size_t)8 << 20, kPinLeast = (size_t)1 << 20;
+struct Copy {
+    void *dst;
+    const void *src;
+    size_t n;
+};
+int readback(hipStream_t st, const std::vector<Copy> &items);
+
 constexpr int kMaxTypes = 64;
 
 struct LJTable {
@@ -60,9 +94,8 @@ struct Ewald {
     double kappa_param = 0, kappa = 0, locut = 0;
     int kmax = 0, nk = 0;
     int sign_mode = 0;    // MH_EWALD_PARITY or MH_EWALD_PHYSICS
-    DBuf k, s, si;        // accepted vectors, reference order
     DBuf ccoef;           // complex coefficient grid c(mx,my,mz) = s + i si, 0 if not kept
-    std::vector<double> hk, hs, hsi;
+    std::vector<double> hk, hs, hsi;  // accepted vectors, reference order
 };
 
 }  // namespace mh

@@ -1571,13 +1571,13 @@ extern "C" int mh_map_build(mh_ctx *ctx, int kind, int precision, double probe_q
             cb.boff[l] = (int32_t *)take(level[l]);
         }
     }
-    if ((rc = map->ptr.alloc(sizeof(int32_t) * nodes))) return fail(rc);
+    if ((rc = pool_take(map->ptr, sizeof(int32_t) * nodes))) return fail(rc);
     int64_t total = 0;
     if ((rc = compact_count(ctx, np, full32, cut, cb, &total)))
         return fail(rc);
     MH_CHECK(total < (1LL << 31), MH_ECAPACITY, "mh_map_build: more than 2^31 tabulated points");
     map->nfsize = total;
-    if ((rc = map->vals.alloc(sizeof(float) * 8 * (total + 1)))) return fail(rc);
+    if ((rc = pool_take(map->vals, sizeof(float) * 8 * (total + 1)))) return fail(rc);
     if ((rc = compact_assign(ctx, np, full32, cb, map->ptr.as<int32_t>(), map->vals.as<float>(), total, map->counts)))
         return fail(rc);
     tcomp.stop();

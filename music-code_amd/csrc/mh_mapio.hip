@@ -67,7 +67,13 @@ int mh_map_destroy(mh_map *map) {
     if (!map) return MH_OK;
     mh_ctx *ctx = map->ctx;
     bool ret = map->retained;
-    if (ctx) (void)hipSetDevice(ctx->device);
+    if (ctx) {
+        (void)hipSetDevice(ctx->device);
+        if (ret && hipDeviceSynchronize() == hipSuccess) {  // as a free would wait
+            pool_give(map->ptr);
+            pool_give(map->vals);
+        }
+    }
     delete map;
     if (ctx && ret) ctx_release(ctx);
     return MH_OK;
@@ -275,26 +281,27 @@ int mh_map_interp(mh_ctx *ctx, const mh_map *map, int n, const double *xyz, doub
     MH_CHECK(n >= 0, MH_EINVAL, "mh_map_interp: n < 0");
     if (n == 0) return MH_OK;
     MH_HIP(hipSetDevice(ctx->device));
-    DBuf dx, de, dok;
+    PoolBuf buf;  // positions, energies, flags
     int rc;
-    if ((rc = dx.alloc(sizeof(double) * 3 * n)) || (rc = de.alloc(sizeof(double) * n)) ||
-        (rc = dok.alloc(n)))
-        return rc;
-    MH_HIP(hipMemcpyAsync(dx.p, xyz, sizeof(double) * 3 * n, hipMemcpyHostToDevice, ctx->stream));
+    if ((rc = buf.take((sizeof(double) * 4 + 1) * (size_t)n))) return rc;
+    double *dx = buf.as<double>(), *de = dx + 3 * (size_t)n;
+    uint8_t *dok = reinterpret_cast<uint8_t *>(de + n);
+    MH_HIP(hipMemcpyAsync(dx, xyz, sizeof(double) * 3 * n, hipMemcpyHostToDevice, ctx->stream));
     SlantCell sc;
     for (int i = 0; i < 9; i++) {
         sc.U[i] = map->U[i];
         sc.S[i] = map->S[i];
     }
-    hipLaunchKernelGGL(k_interp, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, dx.as<double>(),
+    hipLaunchKernelGGL(k_interp, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, dx,
                        map->ptr.as<int32_t>(), map->vals.as<float>(), map->npnts[0], map->npnts[1],
                        map->npnts[2], map->step[0], map->step[1], map->step[2], map->fund_ell[0],
-                       map->fund_ell[1], map->fund_ell[2], factor, map->slanted ? 1 : 0, sc, de.as<double>(),
-                       dok.as<uint8_t>());
+                       map->fund_ell[1], map->fund_ell[2], factor, map->slanted ? 1 : 0, sc, de,
+                       dok);
     MH_HIP(hipGetLastError());
-    MH_HIP(hipMemcpyAsync(e, de.p, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-    MH_HIP(hipMemcpyAsync(ok, dok.p, n, hipMemcpyDeviceToHost, ctx->stream));
+    MH_HIP(hipMemcpyAsync(e, de, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
+    MH_HIP(hipMemcpyAsync(ok, dok, n, hipMemcpyDeviceToHost, ctx->stream));
     MH_HIP(hipStreamSynchronize(ctx->stream));
+    buf.idle = true;
     return MH_OK;
 }
 
