@@ -779,6 +779,124 @@ __global__ void __launch_bounds__(NT, 4) k_nodes32_list(GridP g, const int *__re
     }
 }
 
+// FP64 LJ node values of an orthorhombic cell, the reference's sums in the
+// reference's order and rounding (the stored FP32 values agree to one unit).
+// A block has 8 x 8 columns of 4 NZ nodes, a lane NZ nodes of its column: the
+// folded separations of a staged atom are formed once per axis position of
+// the block, and a lane's nodes share the x, y parts of a pair.  A node stops
+// at its first pair below locut.  Bound by the FP64 issue rate, about 65
+// instructions a pair; with folds and a call of lj_pair64 per pair and node
+// 51^3 nodes of 324 atoms took 187 us.
+template <int NZ>
+__global__ void __launch_bounds__(256, NZ == 4 ? 3 : 4)
+    k_lj_nodes64(GridP g, const PairTab *__restrict__ tab, const double *__restrict__ xyz,
+                 const int *__restrict__ typ, float *__restrict__ out32, double *__restrict__ out64) {
+    constexpr int NZB = 4 * NZ, NE = 16 + NZB, NCH = 32;
+    __shared__ int s_list[SEG];
+    __shared__ int s_w[4];
+    __shared__ double s_s[NCH][NE];
+    __shared__ double4 s_c[NCH];  // A, B, hicut^2, locut^2
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nbx = (g.nx + 7) / 8, nby = (g.ny + 7) / 8;
+    const int x0 = (blockIdx.x % nbx) * 8, y0 = ((blockIdx.x / nbx) % nby) * 8, z0 = (blockIdx.x / (nbx * nby)) * NZB;
+    const int x = x0 + (lane & 7), y = y0 + (lane >> 3), zl = wave * NZ;
+    const double lo[3] = {x0 * g.step[0], y0 * g.step[1], z0 * g.step[2]};
+    const double hi[3] = {min(x0 + 7, g.nx - 1) * g.step[0], min(y0 + 7, g.ny - 1) * g.step[1],
+                          min(z0 + NZB - 1, g.nz - 1) * g.step[2]};
+    double S[NZ][8];
+#pragma unroll
+    for (int i = 0; i < NZ; i++)
+        for (int k = 0; k < 8; k++) S[i][k] = 0.0;
+    unsigned failed = 0;
+#pragma unroll 1
+    for (int seg0 = 0; seg0 < g.natoms; seg0 += SEG) {
+        const int segn = min(SEG, g.natoms - seg0);
+        int cnt = 0;
+        for (int c0 = 0; c0 < segn; c0 += 256) {
+            const int a = seg0 + c0 + tid;
+            bool keep = false;
+            if (c0 + tid < segn) {
+                const double lx = ival_lb(lo[0] - xyz[3 * a], hi[0] - xyz[3 * a], g.full[0]);
+                const double ly = ival_lb(lo[1] - xyz[3 * a + 1], hi[1] - xyz[3 * a + 1], g.full[1]);
+                const double lz = ival_lb(lo[2] - xyz[3 * a + 2], hi[2] - xyz[3 * a + 2], g.full[2]);
+                keep = lx * lx + ly * ly + lz * lz <= g.cull2;
+            }
+            const unsigned long long m = __ballot(keep);
+            if (lane == 0) s_w[wave] = __popcll(m);
+            __syncthreads();
+            int off = cnt;
+            for (int w = 0; w < 4; w++) {
+                if (w < wave) off += s_w[w];
+                cnt += s_w[w];
+            }
+            if (keep) s_list[off + __popcll(m & ((1ull << lane) - 1ull))] = a;
+            __syncthreads();
+        }
+#pragma unroll 1
+        for (int c0 = 0; c0 < cnt; c0 += NCH) {
+            const int m = min(NCH, cnt - c0);
+            for (int w = tid; w < m * NE; w += 256) {
+                const int j = w / NE, e = w - j * NE, a = s_list[c0 + j];
+                const int d = e < 8 ? 0 : (e < 16 ? 1 : 2);
+                const int node = d == 0 ? x0 + e : (d == 1 ? y0 + e - 8 : z0 + e - 16);
+                s_s[j][e] = fold1((double)node * g.step[d] - xyz[3 * a + d], g.full[d]);
+            }
+            if (tid < m) {
+                const int t = typ[s_list[c0 + tid]];
+                s_c[tid] = make_double4(tab->A[t], tab->B[t], tab->h2[t], tab->l2[t]);
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (int j = 0; j < m; j++) {
+                const double sx = s_s[j][lane & 7], sy = s_s[j][8 + (lane >> 3)];
+                const double4 c = s_c[j];
+                const double rxy = __dadd_rn(__dmul_rn(sx, sx), __dmul_rn(sy, sy));
+                const double A12 = __dmul_rn(12.0, c.x), B6 = __dmul_rn(6.0, c.y), A168 = __dmul_rn(168.0, c.x),
+                             B48 = __dmul_rn(48.0, c.y), A2688 = __dmul_rn(-2688.0, c.x), B480 = __dmul_rn(480.0, c.y);
+#pragma unroll
+                for (int i = 0; i < NZ; i++) {
+                    const double sz = s_s[j][16 + zl + i], r2 = __dadd_rn(rxy, __dmul_rn(sz, sz));
+                    const bool in = !(r2 > c.z);
+                    if (in && r2 < c.w) failed |= 1u << i;
+                    // lj_pair64 with every term zero for a pair that does not count
+                    const double r2i = (in && !((failed >> i) & 1u)) ? 1.0 / r2 : 0.0;
+                    const double r6i = __dmul_rn(__dmul_rn(r2i, r2i), r2i), r12i = __dmul_rn(r6i, r6i);
+                    S[i][0] = __dadd_rn(S[i][0], __dsub_rn(__dmul_rn(c.x, r12i), __dmul_rn(c.y, r6i)));
+                    const double f1 = __dmul_rn(__dsub_rn(__dmul_rn(A12, r12i), __dmul_rn(B6, r6i)), r2i);
+                    S[i][1] = __dsub_rn(S[i][1], __dmul_rn(sx, f1));
+                    S[i][2] = __dsub_rn(S[i][2], __dmul_rn(sy, f1));
+                    S[i][3] = __dsub_rn(S[i][3], __dmul_rn(sz, f1));
+                    const double r10i = __dmul_rn(r12i, r2), r16i = __dmul_rn(r10i, r6i);
+                    const double f2 = __dsub_rn(__dmul_rn(A168, r16i), __dmul_rn(B48, r10i));
+                    const double f2x = __dmul_rn(f2, sx);
+                    S[i][4] = __dadd_rn(S[i][4], __dmul_rn(f2x, sy));
+                    S[i][5] = __dadd_rn(S[i][5], __dmul_rn(f2x, sz));
+                    S[i][6] = __dadd_rn(S[i][6], __dmul_rn(__dmul_rn(f2, sy), sz));
+                    const double f3 = __dmul_rn(__dadd_rn(__dmul_rn(A2688, r16i), __dmul_rn(B480, r10i)), r2i);
+                    S[i][7] = __dadd_rn(S[i][7], __dmul_rn(__dmul_rn(__dmul_rn(f3, sx), sy), sz));
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (x >= g.nx || y >= g.ny) return;
+#pragma unroll
+    for (int i = 0; i < NZ; i++) {
+        const int z = z0 + zl + i;
+        if (z >= g.nz) continue;
+        const long long s = ((long long)x * g.ny + y) * g.nz + z;
+        if ((failed >> i) & 1u) S[i][0] = kVeryLrg;
+        float4 *d32 = reinterpret_cast<float4 *>(out32 + 8 * s);
+        d32[0] = make_float4((float)S[i][0], (float)S[i][1], (float)S[i][2], (float)S[i][3]);
+        d32[1] = make_float4((float)S[i][4], (float)S[i][5], (float)S[i][6], (float)S[i][7]);
+        if (out64) {
+            double2 *d64 = reinterpret_cast<double2 *>(out64 + 8 * s);
+            for (int k = 0; k < 4; k++) d64[k] = make_double2(S[i][2 * k], S[i][2 * k + 1]);
+        }
+    }
+}
+
 // ------------------------------------------------ Ewald reciprocal part
 // Parity mode: V(r) = Re sum_k c_k e^{ik.r}, with c_k = s_k + i si_k
 // (ewald_skwaldHOT, ewald.F90:966-1005: realPart = s cos - si sin, which
@@ -1441,7 +1559,14 @@ static int run_nodes(mh_ctx *ctx, int kind, int precision, double probe_q, const
             hipLaunchKernelGGL(k_nodes32<K_LJ>, dim3((unsigned)nblk), dim3(NT), 0, ctx->stream, g, dt,
                                axyz, ctx->type.as<int>(), ctx->q.as<double>(),
                                (const double *)nullptr, full32, o64);
-        else
+        else if (!slanted) {
+            // four nodes a lane where that leaves two waves for each SIMD, else one
+            const bool four = (long long)np[0] * np[1] * np[2] >= 64LL * 4 * 2048;
+            const int nzb = four ? 16 : 4;
+            auto k = four ? k_lj_nodes64<4> : k_lj_nodes64<1>;
+            hipLaunchKernelGGL(k, dim3((unsigned)((long long)nbx * nby * ((np[2] + nzb - 1) / nzb))), dim3(256), 0,
+                               ctx->stream, g, dt, axyz, ctx->type.as<int>(), full32, o64);
+        } else
             hipLaunchKernelGGL(k_nodes64<K_LJ>, dim3((unsigned)nblk), dim3(NT), 0, ctx->stream, g, dt,
                                axyz, ctx->type.as<int>(), ctx->q.as<double>(),
                                (const double *)nullptr, full32, o64);
