@@ -36,19 +36,6 @@ METRIC = "GCMC trial moves/s + map pts/s, FP32-acc vs FP64; p50/p99 request late
 FP32_PEAK_TFLOPS = 157.3  # MI355X FP32 vector, dense
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "map_ewald_real_fp32_charged_50A_hbm_traffic.txt")
-
-
-def measured_traffic():
-    """HBM bytes per launch of the Ewald real-space map kernel from the
-    committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary (copy-calibrated)."""
-    try:
-        for line in open(TRAFFIC_FILE):
-            if line.startswith("traffic_bytes_per_launch:"):
-                return float(line.split(":")[1])
-    except OSError:
-        pass
-    return None
 
 
 def log(*a):
@@ -620,19 +607,18 @@ def main():
     value = 3.0 * nodes / ((t1 - t0) / args.steps)
     log("FP32-acc: %.1f ms/step, %.3e map pts/s; kernel ms: %s" % (ms_per_step, value, ktimes))
 
-    # dominant kernel roofline: Ewald real space in FP32 (documented cutoff)
-    from musichip.hip import real_space_cutoff_default
-    rc = real_space_cutoff_default(cfg["kappa_param"] / np.min(cfg["full_ell"]))
+    # dominant kernel roofline: the FP32 LJ sums (the Ewald real-space time is
+    # near pairs and an interpolated far field, not a sum over pairs in reach)
     vol = float(np.prod(cfg["full_ell"]))
-    pairs_per_node = len(cfg["xyz"]) * (4.0 / 3.0) * np.pi * rc ** 3 / vol
-    flops_launch = 85.0 * pairs_per_node * nodes
-    kname = "nodes32_ewald_real"
+    pairs_per_node = len(cfg["xyz"]) * (4.0 / 3.0) * np.pi * cfg["hicut"] ** 3 / vol
+    flops_launch = 46.0 * pairs_per_node * nodes
+    kname = "nodes32_lj"
     k_ms = ktimes[kname][0] / ktimes[kname][1]
     achieved = flops_launch / (k_ms * 1e-3) / 1e12
     roofline = dict(bound="valu", achieved=round(achieved, 2), peak=FP32_PEAK_TFLOPS, unit="TFLOP/s",
-                    frac=round(achieved / FP32_PEAK_TFLOPS, 4), traffic=measured_traffic(), kernel=kname,
-                    kernel_ms=round(k_ms, 3),
-                    algorithmic="85 FLOP x %.1f pairs/node (r < %.2f A) x %d nodes" % (pairs_per_node, rc, nodes))
+                    frac=round(achieved / FP32_PEAK_TFLOPS, 4), kernel=kname, kernel_ms=round(k_ms, 3),
+                    algorithmic="46 FLOP x %.1f pairs/node (r < %.2f A) x %d nodes" %
+                                (pairs_per_node, cfg["hicut"], nodes))
 
     # FP64 mode: timing, then the stored FP32 values of the FP32-acc maps
     # against those of the FP64 maps (same compaction required)

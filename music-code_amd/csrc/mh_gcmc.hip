@@ -2203,6 +2203,14 @@ int mh_gcmc_create_mix(mh_ctx *ctx, const mh_gcmc_params *spc, int nspc, int nre
     g->slanted = H.slanted != 0;
     g->nk = H.nk;
     g->kstride = g->nk;
+    // FP32 chains beyond one a CU: two waves a chain let two to four chains of
+    // a CU run side by side (270 methane chains, 60 steps: 637 us with four
+    // waves, 365 with two; 200 chains: 380 and 370).  An Ewald step has work
+    // for four waves: the line lies higher (CO2, 270 chains 817 against 1050
+    // us, 400 chains 1340 against 1070).
+    int ncu = 0;
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device);
+    if (g->prec == MH_PREC_FP32 && ncu > 0 && 2LL * nrep > (g->nk ? 3LL : 2LL) * ncu) g->threads = 128;
     if ((rc = g->dP.alloc(sizeof(GDev)))) return rc;
     if ((rc = alloc_replicas(g.get()))) return rc;
     std::vector<int> reps(nrep);
