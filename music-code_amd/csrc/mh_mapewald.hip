@@ -3,21 +3,29 @@
 // Two routes, both in FP64:
 //   * direct: every atom for every node (FP64 maps, the reference's sum);
 //   * near + far (FP32 maps): the grid is cut into tiles of SB^3 nodes.  For
-//     each tile the atoms within R0 = 1.4 a of the tile's box (a = its half
-//     edge), and those whose minimum image changes inside the box, are summed
-//     node by node; the field of the others up to the real-space cutoff is
-//     smooth in the box, so it is summed at FP^3 Chebyshev points only and
-//     interpolated to the nodes axis by axis.  Tiles of twice the edge do the
-//     same for the atoms that are far from them, and pass their polynomial on
-//     to the points of their eight tiles, where it is exact.  The nearest singularity of a
-//     far atom's field lies at 2.4 a from the box centre: the interpolation
-//     converges as 4.6^-FP, 1e-9 of V and 1e-7 of the derivatives for FP = 16,
-//     below the rounding of the FP32 values stored in the map.
+//     each tile the atoms within R0 = 2 a of the tile's box (a = its half
+//     edge; 3.5 A at least), and those whose minimum image changes inside the
+//     box, are summed node by node; the field of the others up to the
+//     real-space cutoff is smooth in the box, so it is summed at FP^3
+//     Chebyshev points only and interpolated to the nodes axis by axis
+//     (polynomial interpolation at Chebyshev points: Trefethen, Approximation
+//     Theory and Approximation Practice, ch. 4 and 8).
+//     Tiles of twice the edge do the same for the atoms that are far from
+//     them, and pass their polynomial on to the points of their eight tiles,
+//     where it is exact.  Along an axis the field of an atom beside the box is
+//     singular at +-2i a: the interpolation converges as (2 + sqrt 5)^-FP =
+//     4.2^-16 = 1e-10 of that atom's V (atoms ahead of the box: 5.8^-16).
+// R0 is what the derivative columns need: against the reference's sums their
+// largest errors were 1.6e-6 of a column's rms (mixed second derivatives) with
+// 1.4 a, where FP32 pair terms leave 5e-8 to 9e-7.  With 2 a, and 3.5 A for the
+// smallest tiles, they are below those of the FP32 pair terms in every column.
 // The reference differentiates erfc exactly but evaluates it with the A&S
-// 7.1.26 fit (ewald.F90:874-916): the far field is therefore carried twice,
-// with the A&S erfc (for V) and with erfc to 1e-9 (whose interpolant is
-// differentiated); the derivative terms differ from the reference's by the
-// fit's 1.5e-7 / r^2 alone.
+// 7.1.26 fit (ewald.F90:874-916), so its derivative sums are not the
+// derivatives of its V.  The far field is therefore carried twice: with the
+// A&S erfc (for V) and as the potential whose first derivative is the
+// reference's term exactly (far_h); its second and third derivatives differ
+// from the reference's by the fit's own slope, 1e-6 / r^3 and / r^4.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -29,9 +37,10 @@ namespace mh {
 
 constexpr int FP = 16;            // Chebyshev points per axis
 constexpr int FPV = FP * FP * FP;
-constexpr int FDEG = 10;          // degree of the erfcx fit
+constexpr int FDEG = 10;          // degree of the far-field fit
 constexpr int FCH = 32;           // far atoms staged per pass
-constexpr double kFarZ0 = 2.4;    // (a + R0) / a
+constexpr double kFarR0 = 2.0;    // R0 / a
+constexpr double kFarR0Min = 3.5; // least R0 (A)
 constexpr double kEwTokcal = 332.064;   // ewald.F90:60
 constexpr double kEwVeryLrg = 1.0e10;   // mapmaker.F90:57
 constexpr double kEwLowCut2 = 1.0e-6;   // ewald.F90:361-362
@@ -49,7 +58,7 @@ struct EwP {
     // bricks with a node near the compaction's cutoff
     float cut, win;
     int bdim[3], *blist, *bflag;
-    double tc, ith;      // erfcx fit variable (t - tc) * ith
+    double tc, ith;      // variable of the far-field fit, (t - tc) * ith
     double fit[FDEG + 1];
 };
 
@@ -188,7 +197,7 @@ __global__ void __launch_bounds__(256) k_ew_shift(EwP p, int ptx, int pty, int p
 }
 
 // Far field at the Chebyshev points: F[split][tile][field][z][y][x], field 0
-// with the A&S erfc, 1 with erfc.  A lane owns the 16 points of one (x, y)
+// with the A&S erfc, 1 the potential of the derivatives (far_h).  A lane owns the 16 points of one (x, y)
 // line.  The Gaussian factor e^{-kappa^2 r^2} is a product of three per-axis
 // factors formed once per atom (48 exponentials for 4096 points), so a point
 // costs r^-1, the A&S t and two polynomials: about 43 FP64 instructions, the
@@ -492,28 +501,62 @@ static void cheb_series(const double *f, int n, double *c) {
     }
 }
 
-// exp(x^2) erfc(x)
-static double erfcx_host(double x) {
-    if (x < 5.0) return std::exp(x * x) * std::erfc(x);
-    // continued fraction x + (1/2)/(x + 1/(x + (3/2)/(x + ...))), from its tail
-    double d = x;
-    for (int k = 60; k >= 1; k--) d = x + 0.5 * k / d;
-    return 1.0 / (d * std::sqrt(M_PI));
+// The potential of the derivative columns: with x = kappa r its pair term is
+// q T(x) / r with T(x) = x * integral over y > x of e(y) / y^2 + c e^{-y^2} / y,
+// e the A&S erfc and c the reference's 2 / sqrt(pi): d/dr of it is the
+// reference's -(u + g) / r.  far_h = e^{x^2} T(x) at the n points x (ascending):
+// eight-point Gauss-Legendre sums from point to point and, beyond the last, on
+// 16 panels in ln y up to e^{-42}.
+static void far_h(const double *x, int n, double *h) {
+    static const double gx[4] = {0.1834346424956498, 0.5255324099163290, 0.7966664774136267, 0.9602898564975363};
+    static const double gw[4] = {0.3626837833783620, 0.3137066458778873, 0.2223810344533745, 0.1012285362903763};
+    const double a[5] = {(double)0.254829592f, (double)-0.284496736f, (double)1.421413741f, (double)-1.453152027f,
+                         (double)1.061405429f};
+    // integral over ln y in [l0, l1] of e^{x0^2} (e(y) / y + c e^{-y^2})
+    auto panel = [&](double l0, double l1, double x0) {
+        double s = 0.0;
+        for (int k = 0; k < 8; k++) {
+            const double y = std::exp(0.5 * (l0 + l1) + 0.5 * (l1 - l0) * (k < 4 ? -gx[k] : gx[k - 4]));
+            const double t = 1.0 / (1.0 + (double)0.3275911f * y);
+            const double e = t * (a[0] + t * (a[1] + t * (a[2] + t * (a[3] + t * a[4]))));
+            s += gw[k & 3] * std::exp(x0 * x0 - y * y) * (e / y + 2.0 * 0.5641896);
+        }
+        return 0.5 * (l1 - l0) * s;
+    };
+    double tail = 0.0;
+    const double xn = x[n - 1], ln0 = std::log(xn), dl = (0.5 * std::log(xn * xn + 42.0) - ln0) / 16;
+    for (int i = 0; i < 16; i++) tail += panel(ln0 + i * dl, ln0 + (i + 1) * dl, xn);
+    for (int i = n - 1; i >= 0; i--) {
+        if (i < n - 1)
+            tail = tail * std::exp(x[i] * x[i] - x[i + 1] * x[i + 1]) + panel(std::log(x[i]), std::log(x[i + 1]), x[i]);
+        h[i] = x[i] * tail;
+    }
 }
 
-// fit of erfcx over [x0, x1] in the variable of the A&S t; false where it
+// fit of far_h over [x0, x1] in the variable of the A&S t; false where it
 // misses 1e-9 (a range too wide for the degree)
-static bool fit_erfcx(double x0, double x1, EwP &p) {
+static bool fit_far(double x0, double x1, EwP &p) {
     const double pp = (double)0.3275911f;
     const double ta = 1.0 / (1.0 + pp * x1), tb = 1.0 / (1.0 + pp * x0);
     p.tc = 0.5 * (ta + tb);
     p.ith = 2.0 / (tb - ta);
-    auto at = [&](double u) { return (1.0 / (p.tc + u / p.ith) - 1.0) / pp; };
-    double f[FDEG + 1], c[FDEG + 1];
-    for (int k = 0; k <= FDEG; k++) f[k] = erfcx_host(at(std::cos(M_PI * (k + 0.5) / (FDEG + 1))));
-    cheb_series(f, FDEG + 1, c);
+    // the interpolation points and 64 others, x ascending (u descending)
+    constexpr int NI = FDEG + 1, NC = 64;
+    struct Pt {
+        double u;
+        int k;  // interpolation point k, or -1
+    } pt[NI + NC];
+    for (int k = 0; k < NI; k++) pt[k] = {std::cos(M_PI * (k + 0.5) / NI), k};
+    for (int k = 0; k < NC; k++) pt[NI + k] = {1.0 - 2.0 * (k + 0.25) / NC, -1};
+    std::sort(pt, pt + NI + NC, [](const Pt &l, const Pt &r) { return l.u > r.u; });
+    double x[NI + NC], h[NI + NC], f[NI], c[NI];
+    for (int k = 0; k < NI + NC; k++) x[k] = (1.0 / (p.tc + pt[k].u / p.ith) - 1.0) / pp;
+    far_h(x, NI + NC, h);
+    for (int k = 0; k < NI + NC; k++)
+        if (pt[k].k >= 0) f[pt[k].k] = h[k];
+    cheb_series(f, NI, c);
     // Chebyshev series to monomials
-    double T[2][FDEG + 1], nx[FDEG + 1];
+    double T[2][NI], nx[NI];
     std::memset(T, 0, sizeof T);
     for (int i = 0; i <= FDEG; i++) p.fit[i] = 0.0;
     T[0][0] = 1.0;
@@ -526,11 +569,10 @@ static bool fit_erfcx(double x0, double x1, EwP &p) {
         std::memcpy(T[1], nx, sizeof nx);
         for (int i = 0; i <= FDEG; i++) p.fit[i] += c[j] * nx[i];
     }
-    for (int k = 0; k <= 64; k++) {
-        const double u = -1.0 + k / 32.0, ex = erfcx_host(at(u));
-        double h = p.fit[FDEG];
-        for (int i = FDEG - 1; i >= 0; i--) h = h * u + p.fit[i];
-        if (!(std::fabs(h - ex) <= 1e-9 * ex)) return false;
+    for (int k = 0; k < NI + NC; k++) {
+        double v = p.fit[FDEG];
+        for (int i = FDEG - 1; i >= 0; i--) v = v * pt[k].u + p.fit[i];
+        if (!(std::fabs(v - h[k]) <= 1e-9 * h[k])) return false;
     }
     return true;
 }
@@ -561,39 +603,83 @@ static void cheb_matrix(int n, const double *xi, double *M, double *Dm) {
     }
 }
 
-// Estimated FP64 instructions per node of the near + far route for tiles of
-// SB^3 nodes (and parents of (2 SB)^3 with two levels): 55 per near pair, 36
-// per far pair and point, 600 for the expansion; the FP32 kernel's direct sum
-// takes 60 per pair and 2500 for its FP64 near pairs.
-static double far_cost(const EwP &p, double rc, double dens, int SB, bool two, double *direct) {
-    const double cell = p.L[0] * p.L[1] * p.L[2];
-    auto level = [&](int sb, double &near, double &far, double within) {
-        double hs = 0.0, vol = 1.0, nodes = 1.0, tiles = 1.0, keep = 1.0, e[3];
-        for (int d = 0; d < 3; d++) {
-            e[d] = (sb - 1) * p.step[d];
-            hs = std::max(hs, 0.5 * e[d]);
-            tiles *= (p.n[d] + sb - 1) / sb;
-            nodes *= p.n[d];
-            vol *= e[d];
-            // atoms whose image changes inside the box: slabs of the box's width
-            if (rc + e[d] >= 0.5 * p.L[d]) keep *= std::max(0.0, 1.0 - e[d] / p.L[d]);
+// volume of a box of edges e grown by r
+static double grown(const double e[3], double r) {
+    return e[0] * e[1] * e[2] + 2.0 * (e[0] * e[1] + e[1] * e[2] + e[0] * e[2]) * r +
+           M_PI * r * r * (e[0] + e[1] + e[2]) + 4.0 / 3.0 * M_PI * r * r * r;
+}
+
+// Expected near and far atoms of a tile of SB^3 nodes with a lattice's uniform
+// density dens: the grown box in closed form, the atoms whose image changes
+// inside the box (and the far ones) by counting the points of a 16^3 grid over
+// the octant of separations of a periodic cell.
+static void tile_counts(const EwP &p, double rc, double dens, int SB, double &near, double &far) {
+    constexpr int G = 16;
+    double m2[3][G], e[3], hs = 0.0;
+    bool cross[3][G];
+    for (int d = 0; d < 3; d++) {
+        e[d] = (SB - 1) * p.step[d];
+        const double h = 0.5 * e[d];
+        hs = std::max(hs, h);
+        for (int i = 0; i < G; i++) {
+            const double s = (i + 0.5) / G * 0.5 * p.L[d], in = std::max(s - h, 0.0);
+            cross[d][i] = s + h >= 0.5 * p.L[d];
+            const double m = cross[d][i] ? std::min(in, std::max(p.L[d] - s - h, 0.0)) : in;
+            m2[d][i] = m * m;
         }
-        const double area = 2.0 * (e[0] * e[1] + e[1] * e[2] + e[0] * e[2]), edges = e[0] + e[1] + e[2];
-        auto grown = [&](double r) {
-            return std::min(dens * cell,
-                            dens * (vol + area * r + M_PI * r * r * edges + 4.0 / 3.0 * M_PI * r * r * r));
-        };
-        const double all = grown(rc);
-        near = grown((kFarZ0 - 1.0) * hs);
-        near += (all - near) * (1.0 - keep);
-        far = std::max(0.0, std::min(all, within) - near) * tiles * FPV / nodes;
-        return near;
-    };
-    double near, far, pnear = 1e300, pfar = 0.0;
-    if (two) level(2 * SB, pnear, pfar, 1e300);
-    level(SB, near, far, pnear);
-    *direct = 2500.0 + 60.0 * std::min(dens * cell, dens * 4.0 / 3.0 * M_PI * rc * rc * rc * 1.25);
-    return 600.0 + 55.0 * near + 36.0 * (far + pfar);
+    }
+    const double r0 = std::max(kFarR0 * hs, kFarR0Min), rc2 = rc * rc, r02 = r0 * r0;
+    int nc = 0, nf = 0;
+    for (int i = 0; i < G; i++)
+        for (int j = 0; j < G; j++)
+            for (int k = 0; k < G; k++) {
+                const double lb2 = m2[0][i] + m2[1][j] + m2[2][k];
+                if (lb2 > rc2 || lb2 <= r02) continue;
+                if (cross[0][i] || cross[1][j] || cross[2][k]) nc++;
+                else nf++;
+            }
+    const double all = dens * p.L[0] * p.L[1] * p.L[2];
+    near = std::min(all, dens * grown(e, r0)) + all * nc / (G * G * G);
+    far = all * nf / (G * G * G);
+}
+
+// Estimated time (us) of the near + far route with tiles of SB^3 nodes (and
+// parents of (2 SB)^3 with two levels), at least `best` where it is not the
+// faster one.  Fitted to 40 maps of 3 to 7 unit cells a side, spacing 0.14 to
+// 0.5 A, alpha 0.2 to 0.45, each with every tile size and level (the largest
+// deviations are a quarter): the choice loses 2 % on average to the fastest
+// one and none of the 40 to the pair kernel.  Tiles of 16 nodes on one level,
+// of 32 and of 40 were never the fastest.
+static double far_time(const EwP &p, double rc, double dens, int SB, bool two, double best) {
+    double near, far, pnear = 0.0, pfar = 0.0, nodes = 1.0, tiles = 1.0, ptiles = 1.0, e[3], hs = 0.0;
+    for (int d = 0; d < 3; d++) {
+        nodes *= p.n[d];
+        tiles *= (p.n[d] + SB - 1) / SB;
+        ptiles *= (p.n[d] + 2 * SB - 1) / (2 * SB);
+        e[d] = (SB - 1) * p.step[d];
+        hs = std::max(hs, 0.5 * e[d]);
+    }
+    const double all = dens * p.L[0] * p.L[1] * p.L[2];
+    // the near atoms of the grown box alone
+    near = std::min(all, dens * grown(e, std::max(kFarR0 * hs, kFarR0Min)));
+    if (256.0 + 2.6e-6 * nodes * (11.0 + near) >= best) return best;
+    tile_counts(p, rc, dens, SB, near, far);
+    if (two) {
+        tile_counts(p, rc, dens, 2 * SB, pnear, pfar);
+        far = std::max(0.0, std::min(near + far, pnear) - near);
+    }
+    return (two ? 390.0 : 256.0) + 2.6e-6 * nodes * (11.0 + near) + 1.14e-6 * FPV * (tiles * far + ptiles * pfar);
+}
+
+// the same of the FP32 pair kernel: the atoms its bricks of bd nodes keep
+static double pair_time(const EwP &p, double rc, double dens, const int bd[3]) {
+    double e[3], nodes = 1.0;
+    for (int d = 0; d < 3; d++) {
+        e[d] = (bd[d] - 1) * p.step[d];
+        nodes *= p.n[d];
+    }
+    const double kept = std::min(dens * p.L[0] * p.L[1] * p.L[2], dens * grown(e, rc));
+    return 117.0 + 1.33e-6 * nodes * (56.0 + kept);
 }
 
 // tiles of SB^3 nodes of the grid in p
@@ -608,7 +694,8 @@ static void set_tiles(EwP &p, int SB) {
         p.ihalf[d] = 1.0 / p.half[d];
         hmax = std::max(hmax, p.half[d]);
     }
-    p.r02 = (kFarZ0 - 1.0) * hmax * (kFarZ0 - 1.0) * hmax;
+    const double r0 = std::max(kFarR0 * hmax, kFarR0Min);
+    p.r02 = r0 * r0;
     // at least 2048 workgroups: eight waves of four on each CU
     p.nsplit = (int)std::max<long long>(1, std::min<long long>(16, (2047 + tiles) / tiles));
 }
@@ -658,7 +745,7 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
     }
     // tile size and levels: the cheapest estimate
     const double dens = p.natoms / (p.L[0] * p.L[1] * p.L[2]);
-    double best = 0.0, direct = 0.0;
+    double best = pair_time(p, rc_real, dens, cb.b);
     int SB = 0;
     bool two = false;
     auto fits = [&](int sb) {  // a box stays well under the single fold of the reference
@@ -666,13 +753,16 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
         for (int d = 0; d < 3; d++) ok = ok && (sb - 1) * step[d] < 0.45 * p.L[d];
         return ok;
     };
-    for (int sb : {16, 24, 32, 40})
-        for (int lv = 0; lv < 2; lv++) {
-            if (!fits(sb << lv)) continue;
-            const double c = far_cost(p, rc_real, dens, sb, lv != 0, &direct);
-            if (SB == 0 || c < best) best = c, SB = sb, two = lv != 0;
-        }
-    if (SB == 0 || best > 0.9 * direct) return MH_OK;
+    const struct {
+        int sb;
+        bool two;
+    } choice[3] = {{24, false}, {24, true}, {16, true}};
+    for (auto &o : choice) {
+        if (!fits(o.sb << (o.two ? 1 : 0))) continue;
+        const double c = far_time(p, rc_real, dens, o.sb, o.two, best);
+        if (c < best) best = c, SB = o.sb, two = o.two;
+    }
+    if (SB == 0) return MH_OK;
     p.rc2 = rc_real * rc_real;
     set_tiles(p, SB);
     EwP pp = p;
@@ -684,7 +774,7 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
     const long long maxlist = 1LL << 27;  // 512 MB of list entries
     if ((tiles + ptiles) * p.natoms > maxlist || tiles > (1LL << 20)) return MH_OK;
     // beyond kappa r = 5.5 the fit runs on under a Gaussian below 1e-13
-    if (!fit_erfcx(p.kappa * std::sqrt(p.r02), std::min(5.5, p.kappa * (rc_real + std::sqrt(diag2))), p)) return MH_OK;
+    if (!fit_far(p.kappa * std::sqrt(p.r02), std::min(5.5, p.kappa * (rc_real + std::sqrt(diag2))), p)) return MH_OK;
     for (int k = 0; k < FP; k++) p.xk[k] = std::cos(M_PI * (k + 0.5) / FP);
     std::memcpy(pp.xk, p.xk, sizeof p.xk);
     std::memcpy(pp.fit, p.fit, sizeof p.fit);
@@ -722,6 +812,7 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
     for (int d = 0; d < 3; d++) p.bdim[d] = cb.b[d];
     cb.list = p.blist;
     MH_HIP(hipMemcpyAsync(dM, M.data(), sizeof(double) * M.size(), hipMemcpyHostToDevice, st));
+    KTimer tfar(ctx, !two ? "ewald_far24" : SB == 24 ? "ewald_far24_two" : "ewald_far16_two");
     int *plist = two ? list + tiles * p.natoms : nullptr, *pcount = two ? count + 2 * tiles : nullptr;
     double *PF = F + (size_t)2 * FPV * tiles * p.nsplit;
     if (two) {
