@@ -66,3 +66,38 @@ def test_far_field_matches_the_direct_sum(edge, cells, spacing, alpha, kmax, rou
         assert e < worst[c]
         if route:
             assert s < mean[c]
+
+
+# cells whose factors e^{-(kappa r)^2} reach down to 1e-33 and to 1e-8
+@pytest.mark.parametrize("edge,spacing,alpha", [(24.0, 0.3, 0.42), (20.0, 0.3, 0.25)])
+def test_direct_sums_against_long_double(edge, spacing, alpha):
+    xyz, q, L = _box(3, (edge,) * 3, 1)
+    ctx = H.Context(0)
+    ctx.upload_framework(xyz, np.zeros(len(xyz), dtype=np.int32), q, L, L)
+    assert ctx.set_ewald(alpha * edge, 3, 1e10) == 0  # no k vectors: the real-space sum alone
+    m = ctx.build_map(H.MH_MAP_EWALD, H.MH_PREC_FP64, spacing, 100.0, keep_full=True)
+    n, v = np.array(m.npnts), m.get_full()[1]
+    m.close()
+    LD = np.longdouble
+    pick = np.random.default_rng(2).choice(len(v), 800, replace=False)
+    pos = np.stack(np.unravel_index(pick, n, order="F"), 1) * (L / (n - 1))
+    a1, a2, a3, a4, a5, p = (LD(np.float32(c)) for c in (0.254829592, -0.284496736, 1.421413741, -1.453152027,
+                                                         1.061405429, 0.3275911))
+    kappa = LD(alpha * edge / edge)
+    d = pos[:, None].astype(LD) - xyz[None].astype(LD)
+    d = np.where(d > 0.5 * edge, d - edge, np.where(d < -0.5 * edge, d + edge, d))
+    r2 = (d * d).sum(-1)
+    x = kappa * np.sqrt(r2)
+    t, ek, w = 1 / (1 + p * x), np.exp(-x * x), 1 / r2
+    u = q * t * (a1 + t * (a2 + t * (a3 + t * (a4 + t * a5)))) * ek / np.sqrt(r2)
+    g = LD(2.0 * 0.5641896) * kappa * q * ek
+    f1, f2 = -(u + g) * w, (3 * (u + g) + 2 * x * x * g) * w * w
+    f3 = -(15 * (u + g) + (10 + 4 * x * x) * x * x * g) * w ** 3
+    X, Y, Z = d[..., 0], d[..., 1], d[..., 2]
+    ref = np.stack([s.sum(1) for s in (u, f1 * X, f1 * Y, f1 * Z, f2 * X * Y, f2 * X * Z, f2 * Y * Z,
+                                       f3 * X * Y * Z)], 1) * LD(332.064)
+    err = np.median((np.abs(v[pick] - ref) / np.abs(ref)).astype(float), 0)
+    print("median relative error per column:", err, flush=True)
+    # a pair sum with IEEE square root and division leaves 5e-16 (V) to 7.4e-16
+    # (third derivative); 5e-15 per pair, one Newton step, leaves 1.1e-15 there
+    assert (err < 8.5e-16).all()
