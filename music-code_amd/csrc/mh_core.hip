@@ -120,21 +120,26 @@ int readback(hipStream_t st, const std::vector<Copy> &items) {
     auto up = [](size_t n) { return (n + 63) / 64 * 64; };
     size_t total = 0, o = 0;
     for (auto &i : items) total += up(i.n);
-    Pool::Block pin;
-    if (int rc = pin_take(total, pin)) return rc;
+    // staged through pinned memory up to the size that is kept; more goes to
+    // the caller's pages (pinning them per call costs more than the waits, and
+    // pinned memory of that size may not be there)
+    Pool::Block pin{nullptr, 0};
+    if (total <= kPinBytes)
+        if (int rc = pin_take(total, pin)) return rc;
     hipError_t e = hipSuccess;
     for (auto &i : items) {
-        if (i.n && e == hipSuccess) e = hipMemcpyAsync((char *)pin.p + o, i.src, i.n, hipMemcpyDeviceToHost, st);
+        if (i.n && e == hipSuccess)
+            e = hipMemcpyAsync(pin.p ? (char *)pin.p + o : i.dst, i.src, i.n, hipMemcpyDeviceToHost, st);
         o += up(i.n);
     }
     const hipError_t w = hipStreamSynchronize(st);
     if (e == hipSuccess) e = w;
     o = 0;
     for (auto &i : items) {
-        if (i.n && e == hipSuccess) std::memcpy(i.dst, (char *)pin.p + o, i.n);
+        if (i.n && pin.p && e == hipSuccess) std::memcpy(i.dst, (char *)pin.p + o, i.n);
         o += up(i.n);
     }
-    pin_give(pin);
+    if (pin.p) pin_give(pin);
     if (e != hipSuccess) {
         set_error(std::string("copy to the host: ") + hipGetErrorString(e));
         return MH_EHIP;

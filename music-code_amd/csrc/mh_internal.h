@@ -63,7 +63,8 @@ struct PoolBuf : DBuf {
 };
 
 // Device arrays read back together: asynchronous copies into pinned memory,
-// one wait, then the caller's arrays (a synchronous copy each costs a wait).
+// one wait, then the caller's arrays (a synchronous copy each costs a wait);
+// more than kPinBytes together goes to the caller's arrays directly.
 // The pinned blocks are the process's (allocating one costs 400 us): each call
 // takes one for itself, at most kPinBlocks of up to kPinBytes are kept, until
 // the last context is gone.

@@ -1,0 +1,87 @@
+"""Calls under allocation limits.  A child process puts a small library ahead
+of libmusic_hip that passes hipMalloc and hipHostMalloc on, or answers "out of
+memory" for requests above a limit; the GPU itself sees ordinary work only."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SHIM = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+size_t shim_dev = (size_t)-1, shim_host = (size_t)-1;   /* largest request let through */
+size_t shim_ndev, shim_nhost, shim_refused;             /* calls since the last reset, refusals */
+static void *sym(const char *n) {
+    static void *h;
+    if (!h) h = dlopen("libamdhip64.so.7", RTLD_NOW);
+    return dlsym(h, n);
+}
+int hipMalloc(void **p, size_t n) {
+    shim_ndev++;
+    if (n > shim_dev) { shim_refused++; *p = 0; return 2; }
+    return ((int (*)(void **, size_t))sym("hipMalloc"))(p, n);
+}
+int hipHostMalloc(void **p, size_t n, unsigned f) {
+    shim_nhost++;
+    if (n > shim_host) { shim_refused++; *p = 0; return 2; }
+    return ((int (*)(void **, size_t, unsigned))sym("hipHostMalloc"))(p, n, f);
+}
+"""
+
+HEAD = """
+import ctypes, sys
+sys.path[:0] = [%r, %r, %r]
+shim = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+var = lambda n: ctypes.c_size_t.in_dll(shim, n)
+import numpy as np
+from musichip import hip as H, hmc as HM, synth
+"""
+
+
+def child(tmp_path, code):
+    src, so = str(tmp_path / "shim.c"), str(tmp_path / "libshim.so")
+    with open(src, "w") as f:
+        f.write(SHIM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", so, src, "-ldl"], check=True)
+    paths = (ROOT, os.path.join(ROOT, "music-code_amd"), os.path.join(ROOT, "tests"))
+    p = subprocess.run([sys.executable, "-u", "-c", HEAD % paths + code, so], capture_output=True, text=True,
+                       timeout=100)
+    print(p.stdout, p.stderr[-2000:], flush=True)
+    assert p.returncode == 0
+    return p.stdout
+
+
+# a 9.6 MB trace, and the same run's in pieces that fit the kept pinned block
+READBACK = """
+import hmc_systems as S
+fw, model = S.framework(), synth.butane_ua()
+ctx = H.Context(0)
+ctx.upload_framework(fw["xyz"], fw["type"], np.zeros(len(fw["xyz"])), S.L16, S.L16)
+maps = {}
+for t, n in enumerate(model["types"]):
+    ctx.set_lj(*synth.lb_table(fw["eps"], fw["sig"], *model["lj"][n], S.HICUT))
+    maps[t] = ctx.build_map(H.MH_MAP_LJ, H.MH_PREC_FP64, S.GRID, 100.0)
+om = [(m.npnts, m.step) + m.get() for m in maps.values()]
+rp = S.place(model, om, 1, 3)
+def batch():
+    b = HM.HmcBatch(ctx, HM.hmc_spec(model, S.L16, S.L16, hicut=S.HICUT), maps, [5, 6, 7, 8], maxN=1)
+    for r in range(4):
+        b.set_config(r, rp)
+        b.set_velocities(r, np.full(rp.shape, 0.1 * r))
+    return b
+var("shim_host").value = 8 << 20
+a, b = batch(), batch()
+whole = a.md(30000)
+parts = np.concatenate([b.md(10000) for _ in range(3)], 1)
+assert var("shim_ndev").value > 0 and var("shim_nhost").value > 0 and var("shim_refused").value == 0
+assert np.array_equal(whole, parts) and np.isfinite(whole).all()
+print("trace of %d bytes" % whole.nbytes)
+"""
+
+
+def test_large_traces_need_no_pinned_memory_of_their_size(tmp_path):
+    assert "trace of 9600000 bytes" in child(tmp_path, READBACK)
