@@ -43,7 +43,7 @@ int pool_take(DBuf &b, size_t bytes) {
         size_t best = q.blocks.size();
         for (size_t i = 0; i < q.blocks.size(); i++) {
             const size_t n = q.blocks[i].n;
-            if (n < bytes || n > 2 * bytes + (1 << 20)) continue;
+            if (n < bytes || n - bytes > bytes / kPoolSlack) continue;
             if (best == q.blocks.size() || n < q.blocks[best].n) best = i;
         }
         if (best < q.blocks.size()) {
@@ -61,7 +61,7 @@ void pool_give(DBuf &b) {
     if (!b.p) return;
     int dev = 0;
     std::lock_guard<std::mutex> lk(g_pool_mu);
-    if (hipGetDevice(&dev) == hipSuccess && g_pools[dev].contexts > 0 && b.n <= kPoolBytes / 2) {
+    if (hipGetDevice(&dev) == hipSuccess && g_pools[dev].contexts > 0 && b.n <= kPoolBytes) {
         Pool &q = g_pools[dev];
         q.blocks.push_back({b.p, b.n});
         q.bytes += b.n;

@@ -45,9 +45,13 @@ struct DBuf {
 // Device blocks kept for the next call of the same kind (hipMalloc and hipFree
 // of a map's arrays cost more than a small map's kernels).  One list per
 // device for every context and thread, at most kPoolBytes in kPoolBlocks
-// blocks, freed with the device's last context and when an allocation fails.
+// blocks (two or three of the largest maps in use, 37 M nodes), freed with the
+// device's last context and when an allocation fails.  A block is at most
+// 1 / kPoolSlack larger than the request it is taken for: maps of one grid
+// differ by a few percent in their records, and what a map holds stays close
+// to what its caller counts.
 // pool_give: the block must be idle (the work that used it waited for).
-constexpr size_t kPoolBytes = (size_t)4 << 30, kPoolBlocks = 16;
+constexpr size_t kPoolBytes = (size_t)2 << 30, kPoolBlocks = 16, kPoolSlack = 16;
 int pool_take(DBuf &b, size_t bytes);
 void pool_give(DBuf &b);
 void pool_ctx(int device, int change);  // contexts of a device: +1 / -1

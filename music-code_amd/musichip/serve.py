@@ -96,10 +96,12 @@ def map_nodes(req):
 
 
 def footprint(req, maxN):
-    """Device bytes a request holds while admitted: map (ptr + records +
-    uncompacted lookup copy) + 3 replicas of state."""
+    """Device bytes a request holds while admitted: map (ptr + records, in
+    blocks up to a sixteenth larger than asked for, + uncompacted lookup copy)
+    + 3 replicas of state.  Idle blocks of closed maps, at most 2 GiB a device
+    and given back when an allocation fails, are not a request's."""
     nodes = map_nodes(req)
-    return nodes * (4 + 32 + 32) + 3 * maxN * 9 * 8 + 4096
+    return nodes * (4 + 32) * 17 // 16 + nodes * 32 + 3 * maxN * 9 * 8 + 4096
 
 
 class MapCache:

@@ -85,3 +85,32 @@ print("trace of %d bytes" % whole.nbytes)
 
 def test_large_traces_need_no_pinned_memory_of_their_size(tmp_path):
     assert "trace of 9600000 bytes" in child(tmp_path, READBACK)
+
+
+# blocks of closed maps: taken again by an equal map, not by one of two thirds
+# their size, which would hold the rest unseen
+POOL = """
+rng = np.random.default_rng(4)
+L = np.full(3, 20.0)
+xyz = synth.lattice_faces(3, 20.0 / 3, rng)
+eps, sig, typ = synth.fw_types(rng, len(xyz))
+ctx = H.Context(0)
+ctx.upload_framework(xyz, typ, np.zeros(len(xyz)), L, L)
+ctx.set_lj(*synth.lb_table(eps, sig, 148.0, 3.73, 9.8))
+def build(h):
+    n = var("shim_ndev").value
+    m = ctx.build_map(H.MH_MAP_LJ, H.MH_PREC_FP64, h, 100.0)
+    new, sizes = var("shim_ndev").value - n, (4 * int(np.prod(m.npnts)), 32 * int(m.nfsize))
+    m.close()
+    return new, sizes
+first, s0 = build(0.17)
+again, s1 = build(0.17)
+less, s2 = build(0.205)
+print(first, again, less, s0, s2)
+assert s1 == s0 and first >= 2 and again == 0
+assert 0.5 < s2[0] / s0[0] < 0.67 and less == 2
+"""
+
+
+def test_kept_blocks_serve_requests_of_their_size_only(tmp_path):
+    child(tmp_path, POOL)
