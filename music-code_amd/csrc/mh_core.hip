@@ -161,6 +161,7 @@ int DBuf::alloc(size_t bytes) {
         e = hipMalloc(&p, bytes);
     }
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the caller's next launch check
         p = nullptr;
         set_error(std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
         return MH_ENOMEM;

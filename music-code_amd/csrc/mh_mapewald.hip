@@ -801,18 +801,16 @@ int ewald_nodes(mh_ctx *ctx, double charge1, double rc_real, const int np[3], co
         for (int k = 0; k < FP; k++) xs[k] = (o * SB + h0 * (1.0 + p.xk[k]) - h1) / h1;
         cheb_matrix(FP, xs, C + o * FP * FP, nullptr);
     }
+    // one scratch block: matrices, far field, lists, counts, bricks (number,
+    // flags, list); where it is not to be had, the pair kernel needs none of it
+    const size_t nF = (size_t)2 * FPV * (tiles * p.nsplit + ptiles * pp.nsplit), nl = (size_t)(tiles + ptiles);
     int rc;
-    int *list = (int *)ws_get(ctx, "ewlist", sizeof(int) * (tiles + ptiles) * p.natoms, &rc);
+    double *dM = (double *)ws_get(ctx, "ewald_far", sizeof(double) * (M.size() + nF) +
+                                  sizeof(int) * (nl * p.natoms + 2 * nl + 2 * (size_t)cb.nbricks + 2), &rc);
+    if (rc == MH_ENOMEM) return MH_OK;
     if (rc) return rc;
-    int *count = (int *)ws_get(ctx, "ewcount", sizeof(int) * 2 * (tiles + ptiles), &rc);
-    if (rc) return rc;
-    double *F = (double *)ws_get(ctx, "ewfar", sizeof(double) * 2 * FPV * (tiles * p.nsplit + ptiles * pp.nsplit), &rc);
-    if (rc) return rc;
-    double *dM = (double *)ws_get(ctx, "ewcheb", sizeof(double) * M.size(), &rc);
-    if (rc) return rc;
-    // number, flags, list
-    int *bl = (int *)ws_get(ctx, "ewbricks", sizeof(int) * (2 * (size_t)cb.nbricks + 2), &rc);
-    if (rc) return rc;
+    double *F = dM + M.size();
+    int *list = (int *)(F + nF), *count = list + nl * p.natoms, *bl = count + 2 * nl;
     p.blist = bl + cb.nbricks;
     p.bflag = bl;
     p.cut = cb.cut;

@@ -114,3 +114,39 @@ assert 0.5 < s2[0] / s0[0] < 0.67 and less == 2
 
 def test_kept_blocks_serve_requests_of_their_size_only(tmp_path):
     child(tmp_path, POOL)
+
+
+# the far field's scratch (165 MB of polynomials here) refused: the pair kernel
+# builds the map
+FAR = """
+rng = np.random.default_rng(11)
+L = np.array([30.0, 26.0, 33.0])
+xyz = synth.lattice_faces(5, 1.0, rng) / 5 * L
+q = rng.uniform(-1.0, 1.0, len(xyz))
+ctx = H.Context(0)
+ctx.upload_framework(xyz, np.zeros(len(xyz), dtype=np.int32), q - q.mean(), L, L)
+ctx.set_ewald(0.4 * 26.0, 3, 1e-10)
+def build(prec):
+    ctx.set_timing(True)
+    m = ctx.build_map(H.MH_MAP_EWALD, prec, 0.16, 100.0)
+    ran = [k for k in ctx.timings() if k.startswith("ewald_far")]
+    ctx.set_timing(False)
+    out = m.get()
+    m.close()
+    return ran, out
+r64, (p64, v64) = build(H.MH_PREC_FP64)
+var("shim_dev").value = 140 << 20
+r32, (p32, v32) = build(H.MH_PREC_FP32)
+refused = var("shim_refused").value
+var("shim_dev").value = 1 << 40
+rfar, (pf, vf) = build(H.MH_PREC_FP32)
+print(r64, r32, refused, rfar)
+assert refused > 0 and r32 == [] and rfar == ["ewald_far24"]
+assert np.array_equal(p32, p64) and np.array_equal(pf, p64)
+scale = np.sqrt((v64.astype(float) ** 2).mean(1))[:, None]
+assert np.abs(v32 - v64).max() / scale.max() < 1e-5 and (np.abs(v32 - vf) < 2e-6 * scale + 1e-6 * np.abs(vf)).all()
+"""
+
+
+def test_far_field_scratch_that_is_not_there(tmp_path):
+    child(tmp_path, FAR)
