@@ -1648,6 +1648,7 @@ struct mh_gcmc {
     size_t lds_bytes = 0;   // dynamic LDS of the launch
     DBuf trial;             // buffers of mh_trial_energy
     std::mutex trial_mu;
+    bool lanes_auto = false;  // plan() chooses threads (until the caller or the autotuner does)
     bool exy_off = false;   // autotuner: e^{i(kx x + ky y)} tables disabled
     bool pool = false;      // slot pool (per-replica system and step budget)
     std::vector<SysHost> sys;
@@ -1817,6 +1818,17 @@ int mh::map_dense(mh_ctx *ctx, mh_map *m, const float **out) {
 // (gfx950: 160 KB per workgroup, one replica per CU), the k-vector register
 // tile, and per system the e^{i(kx x + ky y)} tables behind the molecules;
 // uploads the GDev table.
+//
+// Lanes of a chain, where neither mh_gcmc_set_threads nor the autotuner chose
+// them: 256, but 128 for FP32 chains of one species beyond one a CU (without
+// Ewald) or one and a half, which run side by side on a CU then: 270 methane
+// chains, 60 steps: 637 us with four waves, 365 with two (200 chains: 380 and
+// 370); CO2, 400 chains 1340 against 1070 us (270 chains: 817 against 1050).
+// Only where two chains share the CU's LDS and the k vectors stay in registers
+// if they do with 256 lanes.  Mixtures, cavity bias and slanted cells were not
+// measured and keep 256.  The order of a charged
+// chain's reciprocal sums, hence the last bits of its energies, depends on the
+// number of lanes (FP32 pair energies are added in FP64, without rounding).
 static int plan(mh_gcmc *g) {
     int dev_max = 65536;
     (void)hipDeviceGetAttribute(&dev_max, hipDeviceAttributeMaxSharedMemoryPerBlock, g->ctx->device);
@@ -1831,6 +1843,18 @@ static int plan(mh_gcmc *g) {
     g->nk = nk;
     const long long need = (long long)g->nspc * g->maxN * (3 * g->ns + 6) * (long long)sizeof(double);
     g->ldsmol = !g->ncube && need <= budget;
+    if (g->lanes_auto) {
+        int ncu = 0;
+        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, g->ctx->device);
+        // the tables e^{i(kx x + ky y)} of a charged sorbate lie behind the molecules
+        const GDev &H = g->sys[0].H;
+        const long long tab = H.ewald ? 2LL * H.nsmax * (H.kmax + 1) * (2 * H.kmax + 1) * 8 : 0;
+        const bool two_fit = 2 * ((long long)sizeof(Shared) + (long long)sizeof(GDev) + 1024 + need + tab) <= dev_max;
+        const bool k_fit = !nk || !pick_kpl(nk, 256) || pick_kpl(nk, 128);
+        const bool many = ncu > 0 && 2LL * g->nrep > (nk ? 3LL : 2LL) * ncu;
+        g->threads = g->prec == MH_PREC_FP32 && g->nspc == 1 && !g->ncube && !g->slanted && many && two_fit && k_fit
+                         ? 128 : 256;
+    }
     g->lds_bytes = g->ldsmol ? (size_t)need : 0;
     g->kpl = g->ldsmol ? pick_kpl(nk, g->threads) : 0;
     const long long off = (g->lds_bytes + 255) / 256 * 256, ent = (g->prec == MH_PREC_FP64) ? 16 : 8;
@@ -2203,14 +2227,7 @@ int mh_gcmc_create_mix(mh_ctx *ctx, const mh_gcmc_params *spc, int nspc, int nre
     g->slanted = H.slanted != 0;
     g->nk = H.nk;
     g->kstride = g->nk;
-    // FP32 chains beyond one a CU: two waves a chain let two to four chains of
-    // a CU run side by side (270 methane chains, 60 steps: 637 us with four
-    // waves, 365 with two; 200 chains: 380 and 370).  An Ewald step has work
-    // for four waves: the line lies higher (CO2, 270 chains 817 against 1050
-    // us, 400 chains 1340 against 1070).
-    int ncu = 0;
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device);
-    if (g->prec == MH_PREC_FP32 && ncu > 0 && 2LL * nrep > (g->nk ? 3LL : 2LL) * ncu) g->threads = 128;
+    g->lanes_auto = true;
     if ((rc = g->dP.alloc(sizeof(GDev)))) return rc;
     if ((rc = alloc_replicas(g.get()))) return rc;
     std::vector<int> reps(nrep);
@@ -2250,6 +2267,7 @@ int mh_gcmc_set_threads(mh_gcmc *g, int threads) {
     MH_CHECK(threads >= g->cav_tmax, MH_EINVAL, "mh_gcmc_set_threads: fewer threads than cavity trials");
     MH_HIP(hipSetDevice(g->ctx->device));
     MH_HIP(hipStreamSynchronize(g->ctx->stream));
+    g->lanes_auto = false;
     g->threads = threads;
     return plan(g);
 }
@@ -2548,6 +2566,10 @@ int mh_gcmc_set_cavity(mh_gcmc *g, const mh_cavity *c) {
     g->ncube = nc;
     g->cav_cap = cap;
     g->cav_tmax = tmax;
+    if (g->lanes_auto) {  // the choice for cavity bias, at least one lane a trial
+        g->lanes_auto = false;
+        g->threads = 256;
+    }
     if (g->threads < tmax) g->threads = tmax <= 64 ? 64 : tmax <= 128 ? 128 : tmax <= 256 ? 256 : tmax <= 512 ? 512 : 1024;
     if ((rc = plan(g))) return rc;
     return cav_rebuild(g);
@@ -2622,11 +2644,14 @@ int mh_gcmc_run(mh_gcmc *g, int nsteps) {
         if (int rc = moves_ready(g->sys[0].H, g->nspc, "mh_gcmc_run")) return rc;
     MH_HIP(hipSetDevice(g->ctx->device));
     KTimer t(g->ctx, g->prec == MH_PREC_FP32 ? "gcmc32" : "gcmc64");
+    KTimer tl(g->ctx, g->threads == 64 ? "gcmc_lanes64" : g->threads == 128 ? "gcmc_lanes128"
+                      : g->threads == 256 ? "gcmc_lanes256" : g->threads == 512 ? "gcmc_lanes512" : "gcmc_lanes1024");
     launch_any(g, nsteps);
     MH_HIP(hipGetLastError());
+    tl.stop();
+    t.stop();
     std::vector<int> err(g->nrep);
     const int rrc = readback(g->ctx->stream, {{err.data(), g->err.p, 4 * (size_t)g->nrep}});
-    t.stop();
     if (rrc) return rrc;
     for (int i = 0; i < g->nrep; i++) {
         MH_CHECK(err[i] != 2, MH_ECAPACITY, "mh_gcmc_run: a replica reached maxN molecules");
@@ -2928,6 +2953,7 @@ int mh_gcmc_autotune(mh_gcmc *g, int probe_steps, int *threads_out, int *exy_out
     MH_HIP(hipEventCreate(&e0));
     MH_HIP(hipEventCreate(&e1));
     float best = 1e30f;
+    g->lanes_auto = false;
     int best_t = g->threads;
     bool best_exy_off = g->exy_off;
     for (int t : {64, 128, 256, 512}) {
