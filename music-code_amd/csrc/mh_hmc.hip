@@ -1202,9 +1202,9 @@ int mh_hmc_run(mh_hmc *h, int nmoves) {
     int rc = h->prec == MH_PREC_FP32 ? launch_hmc<MH_PREC_FP32>(h, nmoves) : launch_hmc<MH_PREC_FP64>(h, nmoves);
     if (rc) return rc;
     MH_HIP(hipGetLastError());
+    t.stop();
     std::vector<int> err(h->nrep);
     rc = readback(h->ctx->stream, {{err.data(), h->err.p, 4 * (size_t)h->nrep}});
-    t.stop();
     if (rc) return rc;
     for (int i = 0; i < h->nrep; i++)
         MH_CHECK(err[i] == 0, MH_ESTATE, "mh_hmc_run: a replica's start configuration failed to evaluate");
@@ -1285,9 +1285,9 @@ int mh_hmc_md(mh_hmc *h, int nsteps, double *trace) {
     if (h->prec == MH_PREC_FP32) launch_md<MH_PREC_FP32>(h, nsteps, dtrace.as<double>(), h->lds);
     else launch_md<MH_PREC_FP64>(h, nsteps, dtrace.as<double>(), h->lds);
     MH_HIP(hipGetLastError());
+    t.stop();
     std::vector<int> err(h->nrep);
     rc = readback(h->ctx->stream, {{trace, dtrace.p, 8 * nt}, {err.data(), h->err.p, 4 * (size_t)h->nrep}});
-    t.stop();
     if (rc) return rc;
     dtrace.idle = true;
     for (int i = 0; i < h->nrep; i++)
