@@ -207,7 +207,10 @@ constexpr double kTwoPi = 2.0 * kPi;
 // lane sums added by halving.  Bound by the FP64 sincos of every (k, atom);
 // one lane per candidate over the serial atom loop left 107 waves on the chip
 // for 19^3 candidates (1480 us with 4116 atoms, now 60).  The phase of -k is
-// minus that of k exactly, so its sums are the conjugate.
+// minus that of k exactly, so its sums are the conjugate.  The sums differ from
+// the reference's in their last bits; whether a vector is kept must not: where
+// the rounding of the two orders could decide it (extinct vectors with a cutoff
+// of zero), the atoms are added again in the reference's order.
 __global__ void __launch_bounds__(256) k_sfactor(int kmax, int natoms, const double *__restrict__ xyz,
                           const double *__restrict__ q, double ialpha, double ibeta,
                           double igamma, double ikapPiSq, double iVolPi, double locut,
@@ -237,21 +240,35 @@ __global__ void __launch_bounds__(256) k_sfactor(int kmax, int natoms, const dou
         if (lane < 2) keep[w] = 0;
         return;
     }
-    double sum = 0.0, sumi = 0.0;
-    for (int i = lane; i < natoms; i += 64) {
+    double sum = 0.0, sumi = 0.0, qa = 0.0;
+    auto add = [&](int i) {
         double rdotk = __dadd_rn(__dadd_rn(__dmul_rn(ka2pi, xyz[3 * i]), __dmul_rn(kb2pi, xyz[3 * i + 1])),
                                  __dmul_rn(kg2pi, xyz[3 * i + 2]));
         double sn, cs;
         sincos(rdotk, &sn, &cs);
         sum = __dadd_rn(sum, __dmul_rn(cs, q[i]));
         sumi = __dadd_rn(sumi, __dmul_rn(sn, q[i]));
+    };
+    for (int i = lane; i < natoms; i += 64) {
+        add(i);
+        qa += fabs(q[i]);
     }
     for (int o = 32; o > 0; o >>= 1) {
         sum += __shfl_xor(sum, o);
         sumi += __shfl_xor(sumi, o);
+        qa += __shfl_xor(qa, o);
     }
-    double smag = __dmul_rn(__dmul_rn(factor, factor), __dadd_rn(__dmul_rn(sum, sum), __dmul_rn(sumi, sumi)));
-    const bool kept = !(smag <= locut * 1.0e-3);
+    const double f2 = __dmul_rn(factor, factor), least = locut * 1.0e-3;
+    double smag = __dmul_rn(f2, __dadd_rn(__dmul_rn(sum, sum), __dmul_rn(sumi, sumi)));
+    // n terms of total size qa: two orders of their sum differ by 2 n 2^-53 qa
+    // at most (2^-52 n qa; doubled for the products' own rounding)
+    const double ds = 4.44e-16 * natoms * qa;
+    if (fabs(smag - least) <= f2 * (2.0 * (fabs(sum) + fabs(sumi)) + 2.0 * ds) * ds + 1e-15 * least) {
+        sum = sumi = 0.0;
+        for (int i = 0; i < natoms; i++) add(i);
+        smag = __dmul_rn(f2, __dadd_rn(__dmul_rn(sum, sum), __dmul_rn(sumi, sumi)));
+    }
+    const bool kept = !(smag <= least);
     if (lane >= 2) return;
     keep[w] = kept ? 1 : 0;
     if (!kept) return;
