@@ -2489,8 +2489,12 @@ int mh_gcmc_set_config(mh_gcmc *g, int rep, int n, const double *com, const doub
         MH_HIP(hipMemcpy(g->com.as<double>() + off3, hc.data(), sizeof(double) * 3 * n, hipMemcpyHostToDevice));
         MH_HIP(hipMemcpy(g->ang.as<double>() + off3, ha.data(), sizeof(double) * 3 * n, hipMemcpyHostToDevice));
         MH_HIP(hipMemcpy(g->ctr.as<double>() + off3, hctr.data(), sizeof(double) * 3 * n, hipMemcpyHostToDevice));
-        MH_HIP(hipMemcpy2D(g->pos.as<double>() + offp, sizeof(double) * 3 * g->ns, hp.data(),
-                           sizeof(double) * 3 * ns, sizeof(double) * 3 * ns, n, hipMemcpyHostToDevice));
+        // whole slots in one plain copy (a strided one did not arrive under rocprofv3)
+        std::vector<double> slots(3 * (size_t)g->ns * n, 0.0);
+        for (size_t m = 0; m < (size_t)n; m++)
+            std::memcpy(&slots[3 * m * g->ns], &hp[3 * m * ns], sizeof(double) * 3 * ns);
+        MH_HIP(hipMemcpy(g->pos.as<double>() + offp, slots.data(), sizeof(double) * slots.size(),
+                         hipMemcpyHostToDevice));
     }
     MH_HIP(hipMemcpy(g->N.as<int>() + GSPC * rep + g->sel, &n, sizeof(int), hipMemcpyHostToDevice));
     if (g->ncube) {
@@ -2818,9 +2822,13 @@ int mh_gcmc_get_config(mh_gcmc *g, int rep, int *n, double *com, double *ang, do
     const int ns = g->sys_of(rep).sp[g->sel].ns;
     if (hn && com) MH_HIP(hipMemcpy(com, g->com.as<double>() + off3, sizeof(double) * 3 * hn, hipMemcpyDeviceToHost));
     if (hn && ang) MH_HIP(hipMemcpy(ang, g->ang.as<double>() + off3, sizeof(double) * 3 * hn, hipMemcpyDeviceToHost));
-    if (hn && r)
-        MH_HIP(hipMemcpy2D(r, sizeof(double) * 3 * ns, g->pos.as<double>() + offp, sizeof(double) * 3 * g->ns,
-                           sizeof(double) * 3 * ns, hn, hipMemcpyDeviceToHost));
+    if (hn && r) {
+        std::vector<double> slots(3 * (size_t)g->ns * hn);
+        MH_HIP(hipMemcpy(slots.data(), g->pos.as<double>() + offp, sizeof(double) * slots.size(),
+                         hipMemcpyDeviceToHost));
+        for (size_t m = 0; m < (size_t)hn; m++)
+            std::memcpy(r + 3 * m * ns, &slots[3 * m * g->ns], sizeof(double) * 3 * ns);
+    }
     return MH_OK;
 }
 
