@@ -34,8 +34,19 @@ sys.path.insert(0, os.path.join(ROOT, "music-code_amd"))
 
 METRIC = "GCMC trial moves/s + map pts/s, FP32-acc vs FP64; p50/p99 request latency"
 FP32_PEAK_TFLOPS = 157.3  # MI355X FP32 vector, dense
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "map_charged_50A_hbm_traffic.txt")
 
 
+def measured_traffic():
+    """HBM bytes per launch of the FP32 LJ map kernel from the committed
+    rocprofv3 FETCH_SIZE / WRITE_SIZE summary (copy-calibrated)."""
+    try:
+        for line in open(TRAFFIC_FILE):
+            if line.startswith("traffic_bytes_per_launch:"):
+                return float(line.split(":")[1])
+    except OSError:
+        pass
+    return None
 
 
 def log(*a):
@@ -616,7 +627,8 @@ def main():
     k_ms = ktimes[kname][0] / ktimes[kname][1]
     achieved = flops_launch / (k_ms * 1e-3) / 1e12
     roofline = dict(bound="valu", achieved=round(achieved, 2), peak=FP32_PEAK_TFLOPS, unit="TFLOP/s",
-                    frac=round(achieved / FP32_PEAK_TFLOPS, 4), kernel=kname, kernel_ms=round(k_ms, 3),
+                    frac=round(achieved / FP32_PEAK_TFLOPS, 4), traffic=measured_traffic(), kernel=kname,
+                    kernel_ms=round(k_ms, 3),
                     algorithmic="46 FLOP x %.1f pairs/node (r < %.2f A) x %d nodes" %
                                 (pairs_per_node, cfg["hicut"], nodes))
 
