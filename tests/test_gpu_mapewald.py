@@ -18,23 +18,25 @@ def _box(cells, edge, seed):
     return xyz, q - q.mean(), L
 
 
-# edges, cells per axis, spacing, alpha, kmax, route (None: the FP32 pair
-# kernel): every tile size and level on unequal edges with tiles that do not
-# divide the grid; a cutoff beyond half the edge, so that atoms change their
-# image inside a tile; coarse grids and the smallest one, which take the pairs
-@pytest.mark.parametrize("edge,cells,spacing,alpha,kmax,route", [
-    ((30.0, 26.0, 33.0), 5, 0.16, 0.40, 5, "ewald_far24"),
-    ((30.0, 27.0, 28.5), 5, 0.14, 0.35, 5, "ewald_far16_two"),
-    ((36.0, 36.5, 37.0), 5, 0.14, 0.28, 5, "ewald_far24_two"),
-    ((22.0, 21.3, 21.0), 3, 0.115, 0.25, 4, "ewald_far16_two"),
-    ((33.0, 29.5, 31.7), 4, 0.25, 0.33, 5, None),
-    ((40.0, 40.0, 40.0), 5, 0.41, 0.30, 5, None),
-    ((12.0, 12.0, 12.0), 2, 0.5, 0.40, 3, None),
+# edges, cells per axis, spacing, alpha, kmax, map boxes per axis, route (None:
+# the FP32 pair kernel): every tile size and level on unequal edges with tiles
+# that do not divide the grid; a cutoff beyond half the edge, so that atoms
+# change their image inside a tile; coarse grids and the smallest one, which
+# take the pairs; a map of an eighth of the cell
+@pytest.mark.parametrize("edge,cells,spacing,alpha,kmax,reps,route", [
+    ((30.0, 26.0, 33.0), 5, 0.16, 0.40, 5, 1, "ewald_far24"),
+    ((30.0, 27.0, 28.5), 5, 0.14, 0.35, 5, 1, "ewald_far16_two"),
+    ((36.0, 36.5, 37.0), 5, 0.14, 0.28, 5, 1, "ewald_far24_two"),
+    ((22.0, 21.3, 21.0), 3, 0.115, 0.25, 4, 1, "ewald_far16_two"),
+    ((33.0, 29.5, 31.7), 4, 0.25, 0.33, 5, 1, None),
+    ((40.0, 40.0, 40.0), 5, 0.41, 0.30, 5, 1, None),
+    ((12.0, 12.0, 12.0), 2, 0.5, 0.40, 3, 1, None),
+    ((44.0, 40.0, 42.0), 6, 0.115, 0.36, 5, 2, "ewald_far24_two"),
 ])
-def test_far_field_matches_the_direct_sum(edge, cells, spacing, alpha, kmax, route):
+def test_far_field_matches_the_direct_sum(edge, cells, spacing, alpha, kmax, reps, route):
     xyz, q, L = _box(cells, edge, 11)
     ctx = H.Context(0)
-    ctx.upload_framework(xyz, np.zeros(len(xyz), dtype=np.int32), q, L, L)
+    ctx.upload_framework(xyz, np.zeros(len(xyz), dtype=np.int32), q, L / reps, L)
     ctx.set_ewald(alpha * L.min(), kmax, 1e-10)
     node, ran = {}, {}
     for prec in (H.MH_PREC_FP32, H.MH_PREC_FP64):
